@@ -73,6 +73,14 @@ int decode_n_wg() { return device_cus() * g_wg_per_cu; }
 // with one).
 constexpr int F8_WG_PER_CU = 2;
 
+// Fewer than 4 kv heads leave a workgroup fewer than 4 waves (one per kv
+// head): this many times the ranges, as many to a workgroup (RangeWave<true>),
+// put 4 waves' bytes in flight again.
+int kv_head_ranges(int Hkv) { return Hkv >= 4 || Hkv <= 0 ? 1 : 4 / Hkv; }
+// The most of it that Hq query heads allow (Hkv >= Hq / 8): workspace queries
+// know Hq alone.
+int most_ranges(int Hq) { return kv_head_ranges((Hq + 7) / 8); }
+
 size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // Workspace: [offs: T + 2 ints][part_ms][part_acc].
@@ -471,14 +479,14 @@ int pkv_attn_decode_workspace(int T, int Hq, size_t* bytes) {
     if (T < 0 || Hq <= 0 || !bytes) return PKV_ERR_INVALID;
     // Groups other than 4 query heads per kv head run the verify kernels'
     // records, so the size covers both layouts.
-    *bytes = std::max(decode_layout(T, Hq, decode_n_wg() * F8_WG_PER_CU).total,
-                      decode_layout(T, Hq, decode_n_wg() * F8_WG_PER_CU, true).total);
+    const int n_wg = decode_n_wg() * F8_WG_PER_CU * most_ranges(Hq);
+    *bytes = std::max(decode_layout(T, Hq, n_wg).total, decode_layout(T, Hq, n_wg, true).total);
     return PKV_OK;
 }
 
 int pkv_attn_verify_workspace(int T, int Hq, size_t* bytes) {
     if (T < 0 || Hq <= 0 || !bytes) return PKV_ERR_INVALID;
-    *bytes = decode_layout(T, Hq, decode_n_wg() * F8_WG_PER_CU, true).total;
+    *bytes = decode_layout(T, Hq, decode_n_wg() * F8_WG_PER_CU * most_ranges(Hq), true).total;
     return PKV_OK;
 }
 
@@ -522,6 +530,7 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
     // one token at a time), which read cu.
     // The fused step (bit 4) for G != 4 is the verify kernel with the
     // append fused in, then the verify merge.
+    const bool drafts = phases & 8;
     if (G != 4 && !f8 && (phases & 7)) phases |= 8;
     if ((skip_prompts || (phases & 8)) && !cu) return PKV_ERR_INVALID;
     const bool verify = phases & 8;
@@ -531,14 +540,26 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
     if (!aligned(q, 16) || !aligned(kcache, 16) || !aligned(vcache, 16) || !aligned(qkv, 16) || !aligned(out, 16) ||
         !aligned(workspace, 256))
         return PKV_ERR_INVALID;
-    const int groups = (Hkv + 3) / 4, threads = 64 * std::min(Hkv, 4);
+    const int groups = (Hkv + 3) / 4;
     if (phases & 4) {
         if (!app || !app->k_rows || !app->v_rows || !app->slot_map || !cu) return PKV_ERR_INVALID;
         if (!aligned(app->k_rows, 16) || !aligned(app->v_rows, 16) || app->row_stride % 16 != 0 ||
             app->row_stride < (int64_t)Hkv * pkv::HEAD_DIM * 2)
             return PKV_ERR_INVALID;
     }
-    const int n_wg = decode_n_wg() * (f8 ? F8_WG_PER_CU : 1);
+    const int wgs = decode_n_wg() * (f8 ? F8_WG_PER_CU : 1);
+    // Several ranges to a workgroup (1 or 2 kv heads) from as many tokens on
+    // as give them work: 64 tokens of 512 to 8,192 keys at 4 / 1 heads 83 -> 49
+    // us, at 8 / 2 87 -> 77.5; 128 tokens over E4M3 at 4 / 1 heads 55 -> 44, at
+    // 8 / 2 66 -> 60. Below, the longer search and the merge's extra records
+    // cost what the bytes in flight gain: 48 tokens at 16 / 2 heads 45 -> 47
+    // us, 35 short ones at 4 / 1 24.8 -> 25.5, 1 token at 8 / 2 13.7 -> 14.5.
+    // Draft rows at 2 kv heads, 4 records a piece, lose 4 % at every size.
+    int rpb = T < (f8 && Hkv == 2 ? 128 : 64) || (drafts && Hkv == 2) ? 1 : kv_head_ranges(Hkv);
+    // (a workspace sized otherwise, as the no-allocation array, may not hold
+    // them)
+    if (workspace_bytes < decode_layout(T, Hq, wgs * rpb, verify, G).total) rpb = 1;
+    const int n_wg = wgs * rpb;
     const DecodeLayout lay = decode_layout(T, Hq, n_wg, verify, G);
     if (workspace_bytes < lay.total) return PKV_ERR_INVALID;
     if (fo.mode && T > fo.rows) return PKV_ERR_INVALID;
@@ -563,6 +584,7 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
     p.part_ms = (float*)(ws + lay.ms);
     p.part_acc = (float*)(ws + lay.acc);
     p.n_wg = n_wg;
+    p.nb = wgs;
     p.min_range = g_min_range;
     p.k_rows = app ? (const uint16_t*)app->k_rows : nullptr;
     p.v_rows = app ? (const uint16_t*)app->v_rows : nullptr;
@@ -571,45 +593,37 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
     p.vscale = vscale;
     const int32_t* slot_map = app ? app->slot_map : nullptr;
     if (phases & 5) {
+        const int threads = rpb > 1 ? 256 : 64 * std::min(Hkv, 4);
         hipEvent_t e0 = t_ev_start, e1 = t_ev_stop;
         t_ev_start = t_ev_stop = nullptr;
         using RangeKernel = void (*)(pkv::DecodeParams, const int*, const int*, const int*, const int*, const int*);
         using RangeKernelS =
             void (*)(pkv::DecodeParams, const int*, const int*, const int*, const int*, const int*, const int*);
-        const RangeKernel rk = verify && f8 ? by_group<RangeKernel>(G, pkv::verify_range8_kernel<1>,
-                                                                    pkv::verify_range8_kernel<2>,
-                                                                    pkv::verify_range8_kernel<4>,
-                                                                    pkv::verify_range8_kernel<6>,
-                                                                    pkv::verify_range8_kernel<8>)
-                               : f8 ? by_group<RangeKernel>(G, pkv::decode_range8_kernel<1>,
-                                                            pkv::decode_range8_kernel<2>,
-                                                            pkv::decode_range8_kernel<4>,
-                                                            pkv::decode_range8_kernel<6>,
-                                                            pkv::decode_range8_kernel<8>)
-                                    : nullptr;
-        const RangeKernelS vk = !verify || f8 ? nullptr
-                                : (phases & 4) ? by_group<RangeKernelS>(G, pkv::verify_range_kernel<1, true>,
-                                                                        pkv::verify_range_kernel<2, true>,
-                                                                        pkv::verify_range_kernel<4, true>,
-                                                                        pkv::verify_range_kernel<6, true>,
-                                                                        pkv::verify_range_kernel<8, true>)
-                                               : by_group<RangeKernelS>(G, pkv::verify_range_kernel<1>,
-                                                                        pkv::verify_range_kernel<2>,
-                                                                        pkv::verify_range_kernel<4>,
-                                                                        pkv::verify_range_kernel<6>,
-                                                                        pkv::verify_range_kernel<8>);
+        const bool multi = rpb > 1;
+#define PKV_BY_GROUP(KERNEL, ...)                                                                              \
+    (multi ? by_group(G, pkv::KERNEL<1, __VA_ARGS__ true>, pkv::KERNEL<2, __VA_ARGS__ true>,                   \
+                      pkv::KERNEL<4, __VA_ARGS__ true>, pkv::KERNEL<6, __VA_ARGS__ true>,                      \
+                      pkv::KERNEL<8, __VA_ARGS__ true>)                                                        \
+           : by_group(G, pkv::KERNEL<1, __VA_ARGS__ false>, pkv::KERNEL<2, __VA_ARGS__ false>,                 \
+                      pkv::KERNEL<4, __VA_ARGS__ false>, pkv::KERNEL<6, __VA_ARGS__ false>,                    \
+                      pkv::KERNEL<8, __VA_ARGS__ false>))
+        const RangeKernel rk = !f8       ? nullptr
+                               : verify  ? PKV_BY_GROUP(verify_range8_kernel, )
+                                         : PKV_BY_GROUP(decode_range8_kernel, );
+        const RangeKernelS dk = f8 ? nullptr
+                                : verify ? ((phases & 4) ? PKV_BY_GROUP(verify_range_kernel, true, )
+                                                         : PKV_BY_GROUP(verify_range_kernel, false, ))
+                                : (phases & 4) ? (multi ? pkv::decode_range_kernel<4, true, true>
+                                                        : pkv::decode_range_kernel<4, true, false>)
+                                               : (multi ? pkv::decode_range_kernel<4, false, true>
+                                                        : pkv::decode_range_kernel<4, false, false>);
+#undef PKV_BY_GROUP
         if (rk)
-            hipExtLaunchKernelGGL(rk, dim3(n_wg, groups), dim3(threads), 0, (hipStream_t)stream, e0, e1, 0, p, pos,
+            hipExtLaunchKernelGGL(rk, dim3(wgs, groups), dim3(threads), 0, (hipStream_t)stream, e0, e1, 0, p, pos,
                                   tok_seq, block_table, cu, outs);
-        else if (vk)
-            hipExtLaunchKernelGGL(vk, dim3(n_wg, groups), dim3(threads), 0, (hipStream_t)stream, e0, e1, 0, p, pos,
-                                  tok_seq, block_table, cu, outs, slot_map);
-        else if (phases & 4)
-            hipExtLaunchKernelGGL((pkv::decode_range_kernel<4, true>), dim3(n_wg, groups), dim3(threads), 0,
-                                  (hipStream_t)stream, e0, e1, 0, p, pos, tok_seq, block_table, cu, outs, slot_map);
         else
-            hipExtLaunchKernelGGL((pkv::decode_range_kernel<4, false>), dim3(n_wg, groups), dim3(threads), 0,
-                                  (hipStream_t)stream, e0, e1, 0, p, pos, tok_seq, block_table, cu, outs, slot_map);
+            hipExtLaunchKernelGGL(dk, dim3(wgs, groups), dim3(threads), 0, (hipStream_t)stream, e0, e1, 0, p, pos,
+                                  tok_seq, block_table, cu, outs, slot_map);
         const int st = launch_status();
         if (st != PKV_OK) return st;
     }

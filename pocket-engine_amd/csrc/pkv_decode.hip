@@ -67,7 +67,8 @@ struct DecodeParams {
     int* offs;                // [T + 2]: key offsets, then W and R
     float* part_ms;           // [(T + n_wg) * Hq][2]: max (log2 units), sum
     float* part_acc;          // [(T + n_wg) * Hq][256]
-    int n_wg, min_range;
+    int n_wg, min_range;      // most key ranges, fewest keys of one
+    int nb;                   // workgroups (RangeWave<true>)
     // fused step: the step's new rows (k_rows + t * row_stride, Hkv * 256 each)
     const uint16_t* k_rows;
     const uint16_t* v_rows;
@@ -494,58 +495,87 @@ __device__ __forceinline__ void decode_piece(const DecodeParams& p, const int* _
         piece_body<G, false>(p, bt, lds, t, kvh, j0, j1, L, INT_MAX, 0, epi);
 }
 
+// The waves of a key-range workgroup: a wave per kv head of the workgroup's
+// group of up to 4 (blockIdx.y), for one range, number blockIdx.x. MULTI, for
+// 1 or 2 kv heads: 4 waves that take rpb = 4 / Hkv ranges, p.nb (the grid)
+// apart: one search for all of them, and 4 waves' bytes in flight per
+// workgroup; the first nb ranges, all there are of a short step, still spread
+// over the chip.
+template <bool MULTI>
+struct RangeWave {
+    int heads, rpb, wave, sub, head, kvh, b;
+    __device__ __forceinline__ explicit RangeWave(const DecodeParams& p) {
+        wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        heads = MULTI ? p.Hkv : blockDim.x >> 6;
+        rpb = MULTI ? 4 >> (heads - 1) : 1;
+        sub = MULTI ? wave >> (heads - 1) : 0;
+        head = MULTI ? wave & (heads - 1) : wave;
+        kvh = blockIdx.y * 4 + head;
+        b = MULTI ? blockIdx.x + p.nb * sub : blockIdx.x;  // this wave's range
+    }
+};
+// MULTI: fewest keys of a range (a short one is mostly its start and its
+// record): with 64, 96 sequences of 300 to 5,000 keys at 8 / 1 heads over E4M3
+// took 44.3 us instead of 42.7, with 256, 48 at 4 / 1 heads in bf16 40.7
+// instead of 32.2.
+constexpr int RANGE_KEYS = 128;
+
 // The fused step's append, shared by the fused key-range kernels: block
-// (b, y) writes the step's K and V rows of kv heads 4y .. 4y + 3 for tokens
-// b, b + n_wg, .. into their slots (slot_map; -1 or past the pool: skipped).
-// No range of the launch reads these slots from the cache: keys the step
-// feeds come from the source rows. begin() issues the first token's loads
-// before the range search; finish() stores them after it (the latency
-// overlaps the search) and appends the block's other tokens. Block: 64
-// threads per kv head, one uint4 of K or V per thread and token.
+// (b, y) writes the step's K and V rows of kv heads 4y .. 4y + 3 for the
+// tokens of its ranges' numbers, then those n_wg further, into their slots
+// (slot_map; -1 or past the pool: skipped). No range of the launch reads
+// these slots from the cache: keys the step feeds come from the source rows.
+// begin() issues the first token's loads before the range search; finish()
+// stores them after it (the latency overlaps the search) and appends the
+// block's other tokens. Block: 64 threads per kv head and token, one uint4
+// of K or V per thread and token.
+template <bool MULTI>
 struct StepAppend {
+    int heads, t0, i;  // kv heads, the thread's first token, its uint4 of the row pair
     long slot = -1;
     uint4 val;
-    __device__ __forceinline__ const uint4* src(const DecodeParams& p, int t, int i) const {
-        const int per_row = (blockDim.x >> 6) * HEAD_DIM / 8;  // uint4 per K (or V) row slice
+    __device__ __forceinline__ explicit StepAppend(const RangeWave<MULTI>& w)
+        : heads(w.heads), t0(w.b), i(MULTI ? w.head * 64 + (threadIdx.x & 63) : threadIdx.x) {}
+    __device__ __forceinline__ const uint4* src(const DecodeParams& p, int t) const {
+        const int per_row = heads * HEAD_DIM / 8;  // uint4 per K (or V) row slice
         const bool is_v = i >= per_row;
         return reinterpret_cast<const uint4*>((is_v ? p.v_rows : p.k_rows) + (size_t)t * p.row_stride +
                                               (size_t)blockIdx.y * 4 * HEAD_DIM) +
                (is_v ? i - per_row : i);
     }
-    __device__ __forceinline__ void store(const DecodeParams& p, long s, int i, uint4 v) const {
-        const int per_row = (blockDim.x >> 6) * HEAD_DIM / 8;
+    __device__ __forceinline__ void store(const DecodeParams& p, long s, uint4 v) const {
+        const int per_row = heads * HEAD_DIM / 8;
         const bool is_v = i >= per_row;
         reinterpret_cast<uint4*>((is_v ? p.vc : p.kc) + ((size_t)s * p.Hkv + blockIdx.y * 4) * HEAD_DIM)
             [is_v ? i - per_row : i] = v;
     }
     __device__ __forceinline__ void begin(const DecodeParams& p, const int* __restrict__ slot_map) {
-        const int b = blockIdx.x;
-        if (b < p.T) {
-            slot = slot_map[b];
-            val = *src(p, b, threadIdx.x);
+        if (t0 < p.T) {
+            slot = slot_map[t0];
+            val = *src(p, t0);
         }
     }
     __device__ __forceinline__ void finish(const DecodeParams& p, const int* __restrict__ slot_map) const {
-        const int b = blockIdx.x, tid = threadIdx.x;
         const long cap = p.num_blocks * PAGE;
-        if (slot >= 0 && slot < cap) store(p, slot, tid, val);
-        for (int t = b + p.n_wg; t < p.T; t += p.n_wg) {
+        if (slot >= 0 && slot < cap) store(p, slot, val);
+        for (int t = t0 + p.n_wg; t < p.T; t += p.n_wg) {
             const long s = slot_map[t];
-            if (s >= 0 && s < cap) store(p, s, tid, *src(p, t, tid));
+            if (s >= 0 && s < cap) store(p, s, *src(p, t));
         }
     }
 };
 
-// The workgroup's key range [start, end) of the flattened key space (keys
-// of token t: lenf(t)), cut into equal ranges of R = max(min_range,
+// The wave's key range [start, end) of the flattened key space (keys of token
+// t: lenf(t)), cut into at most p.n_wg equal ranges of R >= max(min_range,
 // ceil(W / n_wg)) keys, and the token t0 holding key `start` at offset off0.
-// Workgroup (0, 0) also writes offs[t] (exclusive offsets), offs[T] = W and
-// offs[T + 1] = R for the merge. For T <= block size one scan serves both;
-// otherwise a first pass totals W and a second finds the offsets. Returns
-// false (for the whole workgroup) when the range is empty.
-template <class LenF>
-__device__ __forceinline__ bool find_range(const DecodeParams& p, LenF lenf, int* sh_scan, int* sh_t0, int& start,
-                                           int& end, int& t0, int& off0) {
+// The first workgroup also writes offs[t] (exclusive offsets), offs[T] = W
+// and offs[T + 1] = R for the merge. For T <= block size one scan serves
+// both; otherwise a first pass totals W and a second finds the offsets.
+// Called by the whole workgroup; returns false for a wave (or the whole
+// workgroup) whose range is empty. sh_t0: 2 ints per range of the workgroup.
+template <bool MULTI, class LenF>
+__device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWave<MULTI>& rw, LenF lenf, int* sh_scan,
+                                           int* sh_t0, int& start, int& end, int& t0, int& off0) {
     const int T = p.T, nthr = blockDim.x, tid = threadIdx.x, b = blockIdx.x;
     const bool writer = b == 0 && blockIdx.y == 0;
     const bool one = T <= nthr;
@@ -563,23 +593,39 @@ __device__ __forceinline__ bool find_range(const DecodeParams& p, LenF lenf, int
         }
     }
     W = __builtin_amdgcn_readfirstlane(W);  // block-uniform: keep it in scalar registers
-    const int R = max(p.min_range, (W + p.n_wg - 1) / p.n_wg);
-    start = b * R;
-    end = min(W, start + R);
+    int R = max(p.min_range, (W + p.n_wg - 1) / p.n_wg);
+    if constexpr (MULTI) R = max(R, min(RANGE_KEYS, (W + p.nb - 1) / p.nb));
+    // MULTI: the workgroup's k-th range starts at key at(k) (W: past the last;
+    // n_wg R can pass the int range)
+    auto at = [&](int k) {
+        const unsigned long s = (unsigned long)(unsigned)(b + k * p.nb) * (unsigned)R;
+        return __builtin_amdgcn_readfirstlane(s < (unsigned long)W ? (int)s : W);
+    };
+    const int first = MULTI ? at(0) : b * R, last = MULTI ? at(rw.rpb - 1) : first;
+    start = MULTI ? at(rw.sub) : first;
+    end = MULTI ? min(W, start + min(W, R)) : min(W, start + R);
     if (writer && tid == 0) {
         p.offs[T] = W;
         p.offs[T + 1] = R;
     }
+    // token t at `off` with L keys: the workgroup's ranges that start in it
+    auto mark = [&](int t, int off, int L) {
+        if (L <= 0) return;
+        for (int k = 0; k < (MULTI ? rw.rpb : 1); k++) {
+            const int s = MULTI ? at(k) : first;
+            if (off <= s && s < off + L) {
+                sh_t0[2 * k] = t;
+                sh_t0[2 * k + 1] = off;
+            }
+        }
+    };
     if (one) {
         if (tid < T) {
             if (writer) p.offs[tid] = myoff;
-            if (myL > 0 && myoff <= start && start < myoff + myL) {
-                sh_t0[0] = tid;
-                sh_t0[1] = myoff;
-            }
+            mark(tid, myoff, myL);
         }
     } else {
-        if (start >= W && b != 0) return false;
+        if (first >= W && b != 0) return false;
         int run = 0;
         for (int base = 0; base < T; base += nthr) {
             const int t = base + tid;
@@ -588,45 +634,46 @@ __device__ __forceinline__ bool find_range(const DecodeParams& p, LenF lenf, int
             const int off = run + block_scan(L, sh_scan, tot);
             if (t < T) {
                 if (writer) p.offs[t] = off;
-                if (L > 0 && off <= start && start < off + L) {
-                    sh_t0[0] = t;
-                    sh_t0[1] = off;
-                }
+                mark(t, off, L);
             }
             run += tot;
-            if (b != 0 && run > start) break;  // uniform: every thread has the same run
+            if (b != 0 && run > last) break;  // uniform: every thread has the same run
         }
     }
-    if (start >= W) return false;
+    if (first >= W) return false;
     __syncthreads();
-    t0 = __builtin_amdgcn_readfirstlane(sh_t0[0]);
-    off0 = __builtin_amdgcn_readfirstlane(sh_t0[1]);
+    if (MULTI && start >= W) return false;
+    t0 = __builtin_amdgcn_readfirstlane(sh_t0[2 * rw.sub]);
+    off0 = __builtin_amdgcn_readfirstlane(sh_t0[2 * rw.sub + 1]);
     return true;
 }
 
 // Key-range kernel (FUSED = false) or fused step kernel (FUSED = true): one
 // workgroup per key range and group of up to 4 kv heads (blockIdx.y), a wave
-// per kv head. Block: 64 * min(Hkv, 4) threads (the host rejects Hkv > 4 that
-// is not a multiple of 4).
-template <int G, bool FUSED>
+// per kv head, or with MULTI per 4 / Hkv ranges (RangeWave). Block: 64 *
+// min(Hkv, 4) threads, MULTI 256 (the host rejects Hkv > 4 that is not a
+// multiple of 4).
+template <int G, bool FUSED, bool MULTI>
 __global__ void __launch_bounds__(256, 1)
     decode_range_kernel(DecodeParams p, const int* __restrict__ pos, const int* __restrict__ tok_seq,
                         const int* __restrict__ block_table, const int* __restrict__ cu,
                         const int* __restrict__ outs, const int* __restrict__ slot_map) {
     __shared__ int sh_scan[16];
-    __shared__ int sh_t0[2];
+    __shared__ int sh_t0[8];
     __shared__ WaveLds<G> sh_w[4];
     // pos and tok_seq of every token (T <= block size): a piece's sequence,
     // first row and first position come from LDS, not from dependent global
     // loads at every piece start.
     __shared__ int sh_pos[256], sh_seq[256];
-    const int T = p.T, nthr = blockDim.x, tid = threadIdx.x, b = blockIdx.x;
+    const int T = p.T, nthr = blockDim.x, tid = threadIdx.x;
+    const RangeWave<MULTI> rw(p);
+    const int b = rw.b;
     const bool tab = T <= nthr;
-    StepAppend app;
+    StepAppend<MULTI> app(rw);
     if constexpr (FUSED) app.begin(p, slot_map);
     int start, end, t0, off0;
     const bool any = find_range(
-        p,
+        p, rw,
         [&](int t) {
             const int L = decode_len(t, pos, tok_seq, cu, p.skip_prompts, outs, p.spec);
             if (tab) {
@@ -638,7 +685,7 @@ __global__ void __launch_bounds__(256, 1)
         sh_scan, sh_t0, start, end, t0, off0);
     if constexpr (FUSED) app.finish(p, slot_map);
     if (!any) return;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kvh = blockIdx.y * 4 + wave;
+    const int wave = rw.wave, kvh = rw.kvh;
     int t = t0, off = off0;
     while (off < end && t < T) {
         const int L = !tab || p.skip_prompts ? decode_len(t, pos, tok_seq, cu, p.skip_prompts, outs, p.spec)
@@ -684,9 +731,12 @@ template __global__ void decode_merge_kernel<1>(DecodeParams);
 template __global__ void decode_merge_kernel<4>(DecodeParams);
 template __global__ void decode_merge_kernel<16>(DecodeParams);
 
-template __global__ void decode_range_kernel<4, false>(DecodeParams, const int*, const int*, const int*, const int*,
-                                                       const int*, const int*);
-template __global__ void decode_range_kernel<4, true>(DecodeParams, const int*, const int*, const int*, const int*,
-                                                      const int*, const int*);
+#define PKV_DECODE_RANGE(FUSED, MULTI)                                                                             \
+    template __global__ void decode_range_kernel<4, FUSED, MULTI>(DecodeParams, const int*, const int*, const int*, \
+                                                                  const int*, const int*, const int*);
+PKV_DECODE_RANGE(false, false)
+PKV_DECODE_RANGE(false, true)
+PKV_DECODE_RANGE(true, false)
+PKV_DECODE_RANGE(true, true)
 
 }  // namespace pkv

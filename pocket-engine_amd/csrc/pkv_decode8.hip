@@ -304,22 +304,24 @@ struct DecodeEpi8 {
 
 // Key-range kernel over the E4M3 cache: decode_range_kernel<4, false>'s
 // ranges and records with piece_body8 inside (G query heads per kv head).
-// Grid (n_wg, ceil(Hkv / 4)), 64 * min(Hkv, 4) threads; two workgroups per
-// CU (at most 256 VGPRs).
-template <int G>
+// Grid (workgroups, ceil(Hkv / 4)), 64 * min(Hkv, 4) threads (MULTI: 256,
+// RangeWave); two workgroups per CU (at most 256 VGPRs).
+template <int G, bool MULTI>
 __global__ void __launch_bounds__(256, 2)
     decode_range8_kernel(DecodeParams p, const int* __restrict__ pos, const int* __restrict__ tok_seq,
                          const int* __restrict__ block_table, const int* __restrict__ cu,
                          const int* __restrict__ outs) {
     __shared__ int sh_scan[16];
-    __shared__ int sh_t0[2];
+    __shared__ int sh_t0[8];
     __shared__ WaveLds8 sh_w[4];
     __shared__ int sh_pos[256], sh_seq[256];
-    const int T = p.T, nthr = blockDim.x, tid = threadIdx.x, b = blockIdx.x;
+    const int T = p.T, nthr = blockDim.x, tid = threadIdx.x;
+    const RangeWave<MULTI> rw(p);
+    const int b = rw.b;
     const bool tab = T <= nthr;
     int start, end, t0, off0;
     const bool any = find_range(
-        p,
+        p, rw,
         [&](int t) {
             const int L = decode_len(t, pos, tok_seq, cu, p.skip_prompts, outs, p.spec);
             if (tab) {
@@ -330,7 +332,7 @@ __global__ void __launch_bounds__(256, 2)
         },
         sh_scan, sh_t0, start, end, t0, off0);
     if (!any) return;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kvh = blockIdx.y * 4 + wave;
+    const int wave = rw.wave, kvh = rw.kvh;
     int t = t0, off = off0;
     while (off < end && t < T) {
         const int L = !tab || p.skip_prompts ? decode_len(t, pos, tok_seq, cu, p.skip_prompts, outs, p.spec)

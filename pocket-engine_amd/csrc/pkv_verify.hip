@@ -290,25 +290,27 @@ struct VerifyEpi {
 // FUSED (the fused decode step for groups other than 4): the kernel also
 // appends the step's K/V rows (StepAppend) and reads the keys the step feeds
 // from those source rows (verify_piece), so no range waits for a write.
-template <int G, bool FUSED = false>
+template <int G, bool FUSED, bool MULTI>
 __global__ void __launch_bounds__(256, 2)
     verify_range_kernel(DecodeParams p, const int* __restrict__ pos, const int* __restrict__ tok_seq,
                         const int* __restrict__ block_table, const int* __restrict__ cu,
                         const int* __restrict__ outs, const int* __restrict__ slot_map) {
     constexpr int NR = vf_rows(G);
     __shared__ int sh_scan[16];
-    __shared__ int sh_t0[2];
+    __shared__ int sh_t0[8];
     __shared__ __align__(16) uint16_t sh_v[4][VF_LDS];
-    const int T = p.T, nthr = blockDim.x, tid = threadIdx.x, b = blockIdx.x;
-    StepAppend app;
+    const int T = p.T;
+    const RangeWave<MULTI> rw(p);
+    const int b = rw.b;
+    StepAppend<MULTI> app(rw);
     if constexpr (FUSED) app.begin(p, slot_map);
     int nr, start, end, t0, off0;
     const bool any = find_range(
-        p, [&](int t) { return seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr); }, sh_scan,
+        p, rw, [&](int t) { return seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr); }, sh_scan,
         sh_t0, start, end, t0, off0);
     if constexpr (FUSED) app.finish(p, slot_map);
     if (!any) return;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kvh = blockIdx.y * 4 + wave;
+    const int wave = rw.wave, kvh = rw.kvh;
     int t = t0, off = off0;
     while (off < end && t < T) {
         const int Ls =
@@ -341,23 +343,25 @@ __global__ void __launch_bounds__(256, 2)
 
 // The same over an E4M3 cache with the E4M3 decode body (two pages per
 // step, both products on MFMA, 16 columns = rows x query heads): grid
-// (n_wg, ceil(Hkv / 4)) with two workgroups per CU (at most 256 VGPRs).
-template <int G>
+// (workgroups, ceil(Hkv / 4)) with two workgroups per CU (at most 256 VGPRs).
+template <int G, bool MULTI>
 __global__ void __launch_bounds__(256, 2)
     verify_range8_kernel(DecodeParams p, const int* __restrict__ pos, const int* __restrict__ tok_seq,
                          const int* __restrict__ block_table, const int* __restrict__ cu,
                          const int* __restrict__ outs) {
     constexpr int NR = vf_rows(G);
     __shared__ int sh_scan[16];
-    __shared__ int sh_t0[2];
+    __shared__ int sh_t0[8];
     __shared__ WaveLds8 sh_w8[4];
-    const int T = p.T, tid = threadIdx.x, b = blockIdx.x;
+    const int T = p.T;
+    const RangeWave<MULTI> rw(p);
+    const int b = rw.b;
     int nr, start, end, t0, off0;
     if (!find_range(
-            p, [&](int t) { return seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr); }, sh_scan,
+            p, rw, [&](int t) { return seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr); }, sh_scan,
             sh_t0, start, end, t0, off0))
         return;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kvh = blockIdx.y * 4 + wave;
+    const int wave = rw.wave, kvh = rw.kvh;
     int t = t0, off = off0;
     while (off < end && t < T) {
         const int Ls =
