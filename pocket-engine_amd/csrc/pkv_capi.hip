@@ -88,13 +88,12 @@ struct DecodeLayout {
     size_t offs, ms, acc, total;
 };
 
-// Partial rows: (T + n_wg) indices x Hq heads, times 4 query rows per index
-// for the verify kernel.
-// verify: the verify kernels' records, one per segment row (vf_rows(G); the
-// workspace queries, which do not know G, size for the most, VF_ROWS).
-DecodeLayout decode_layout(int T, int Hq, int n_wg, bool verify = false, int G = 0) {
+// Partial rows: (T + n_wg) indices x Hq heads x nr, 1 for the decode kernels
+// and the rows of a segment for the verify kernels (the workspace queries,
+// which do not know G, size for the most, VF_ROWS).
+DecodeLayout decode_layout(int T, int Hq, int n_wg, int nr = 1) {
     DecodeLayout d;
-    const size_t rows = (size_t)(T + n_wg) * Hq * (verify ? (G > 0 ? pkv::vf_rows(G) : pkv::VF_ROWS) : 1);
+    const size_t rows = (size_t)(T + n_wg) * Hq * nr;
     d.offs = 0;
     d.ms = round_up((size_t)(T + 2) * 4, 256);
     d.acc = d.ms + round_up(rows * 2 * 4, 256);
@@ -480,13 +479,13 @@ int pkv_attn_decode_workspace(int T, int Hq, size_t* bytes) {
     // Groups other than 4 query heads per kv head run the verify kernels'
     // records, so the size covers both layouts.
     const int n_wg = decode_n_wg() * F8_WG_PER_CU * most_ranges(Hq);
-    *bytes = std::max(decode_layout(T, Hq, n_wg).total, decode_layout(T, Hq, n_wg, true).total);
+    *bytes = std::max(decode_layout(T, Hq, n_wg).total, decode_layout(T, Hq, n_wg, pkv::VF_ROWS).total);
     return PKV_OK;
 }
 
 int pkv_attn_verify_workspace(int T, int Hq, size_t* bytes) {
     if (T < 0 || Hq <= 0 || !bytes) return PKV_ERR_INVALID;
-    *bytes = decode_layout(T, Hq, decode_n_wg() * F8_WG_PER_CU * most_ranges(Hq), true).total;
+    *bytes = decode_layout(T, Hq, decode_n_wg() * F8_WG_PER_CU * most_ranges(Hq), pkv::VF_ROWS).total;
     return PKV_OK;
 }
 
@@ -556,11 +555,17 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
     // us, 35 short ones at 4 / 1 24.8 -> 25.5, 1 token at 8 / 2 13.7 -> 14.5.
     // Draft rows at 2 kv heads, 4 records a piece, lose 4 % at every size.
     int rpb = T < (f8 && Hkv == 2 ? 128 : 64) || (drafts && Hkv == 2) ? 1 : kv_head_ranges(Hkv);
-    // (a workspace sized otherwise, as the no-allocation array, may not hold
-    // them)
-    if (workspace_bytes < decode_layout(T, Hq, wgs * rpb, verify, G).total) rpb = 1;
+    // Rows per segment and its records: vf_rows(G), which the 16 columns of one
+    // MFMA hold; draft rows at G = 6 or 8 take two column blocks for 4 rows to
+    // a page pass. (A workspace sized otherwise, as the no-allocation array,
+    // may not hold what is wanted.)
+    int nr = verify ? pkv::vf_rows(G) : 1;
+    if (drafts && !f8 && G >= 6 &&
+        workspace_bytes >= decode_layout(T, Hq, wgs * rpb, pkv::VF_ROWS).total)
+        nr = pkv::VF_ROWS;
+    if (workspace_bytes < decode_layout(T, Hq, wgs * rpb, nr).total) rpb = 1;
     const int n_wg = wgs * rpb;
-    const DecodeLayout lay = decode_layout(T, Hq, n_wg, verify, G);
+    const DecodeLayout lay = decode_layout(T, Hq, n_wg, nr);
     if (workspace_bytes < lay.total) return PKV_ERR_INVALID;
     if (fo.mode && T > fo.rows) return PKV_ERR_INVALID;
     pkv::DecodeParams p;
@@ -600,24 +605,34 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
         using RangeKernelS =
             void (*)(pkv::DecodeParams, const int*, const int*, const int*, const int*, const int*, const int*);
         const bool multi = rpb > 1;
-#define PKV_BY_GROUP(KERNEL, ...)                                                                              \
-    (multi ? by_group(G, pkv::KERNEL<1, __VA_ARGS__ true>, pkv::KERNEL<2, __VA_ARGS__ true>,                   \
-                      pkv::KERNEL<4, __VA_ARGS__ true>, pkv::KERNEL<6, __VA_ARGS__ true>,                      \
-                      pkv::KERNEL<8, __VA_ARGS__ true>)                                                        \
-           : by_group(G, pkv::KERNEL<1, __VA_ARGS__ false>, pkv::KERNEL<2, __VA_ARGS__ false>,                 \
-                      pkv::KERNEL<4, __VA_ARGS__ false>, pkv::KERNEL<6, __VA_ARGS__ false>,                    \
-                      pkv::KERNEL<8, __VA_ARGS__ false>))
+#define PKV_BY_GROUP(KERNEL)                                                                                   \
+    (multi ? by_group(G, pkv::KERNEL<1, true>, pkv::KERNEL<2, true>, pkv::KERNEL<4, true>,                     \
+                      pkv::KERNEL<6, true>, pkv::KERNEL<8, true>)                                              \
+           : by_group(G, pkv::KERNEL<1, false>, pkv::KERNEL<2, false>, pkv::KERNEL<4, false>,                  \
+                      pkv::KERNEL<6, false>, pkv::KERNEL<8, false>))
+#define PKV_VERIFY_M(FUSED, MULTI)                                                                             \
+    by_group(G, pkv::verify_range_kernel<1, 4, FUSED, MULTI>, pkv::verify_range_kernel<2, 4, FUSED, MULTI>,    \
+             pkv::verify_range_kernel<4, 4, FUSED, MULTI>, pkv::verify_range_kernel<6, 2, FUSED, MULTI>,       \
+             pkv::verify_range_kernel<8, 2, FUSED, MULTI>)
+#define PKV_VERIFY(FUSED) (multi ? PKV_VERIFY_M(FUSED, true) : PKV_VERIFY_M(FUSED, false))
         const RangeKernel rk = !f8       ? nullptr
-                               : verify  ? PKV_BY_GROUP(verify_range8_kernel, )
-                                         : PKV_BY_GROUP(decode_range8_kernel, );
-        const RangeKernelS dk = f8 ? nullptr
-                                : verify ? ((phases & 4) ? PKV_BY_GROUP(verify_range_kernel, true, )
-                                                         : PKV_BY_GROUP(verify_range_kernel, false, ))
+                               : verify  ? PKV_BY_GROUP(verify_range8_kernel)
+                                         : PKV_BY_GROUP(decode_range8_kernel);
+        RangeKernelS dk = f8 ? nullptr
+                                : verify ? ((phases & 4) ? PKV_VERIFY(true)
+                                                         : PKV_VERIFY(false))
                                 : (phases & 4) ? (multi ? pkv::decode_range_kernel<4, true, true>
                                                         : pkv::decode_range_kernel<4, true, false>)
                                                : (multi ? pkv::decode_range_kernel<4, false, true>
                                                         : pkv::decode_range_kernel<4, false, false>);
+#undef PKV_VERIFY
+#undef PKV_VERIFY_M
 #undef PKV_BY_GROUP
+        if (dk && nr > pkv::vf_rows(G))
+            dk = G == 6 ? (multi ? pkv::verify_range_kernel<6, 4, false, true>
+                                 : pkv::verify_range_kernel<6, 4, false, false>)
+                        : (multi ? pkv::verify_range_kernel<8, 4, false, true>
+                                 : pkv::verify_range_kernel<8, 4, false, false>);
         if (rk)
             hipExtLaunchKernelGGL(rk, dim3(wgs, groups), dim3(threads), 0, (hipStream_t)stream, e0, e1, 0, p, pos,
                                   tok_seq, block_table, cu, outs);
@@ -631,7 +646,7 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
         // waves per (row, head) block chosen as for decode_merge_kernel below
         using MergeKernel = void (*)(pkv::DecodeParams, const int*, const int*, const int*, const int*);
         const int nw = (int64_t)T * Hq < device_cus() ? 16 : (int64_t)T + n_wg <= 12 * (int64_t)T ? 1 : 4;
-        const bool r4 = pkv::vf_rows(G) == 4;
+        const bool r4 = nr == 4;
         const MergeKernel mk = nw == 16 ? (r4 ? pkv::verify_merge_kernel<4, 16> : pkv::verify_merge_kernel<2, 16>)
                                : nw == 1 ? (r4 ? pkv::verify_merge_kernel<4, 1> : pkv::verify_merge_kernel<2, 1>)
                                          : (r4 ? pkv::verify_merge_kernel<4, 4> : pkv::verify_merge_kernel<2, 4>);
@@ -756,9 +771,10 @@ int pkv_attn_decode_step_noalloc(const void* k_rows, const void* v_rows, int64_t
                                  const int32_t* cu, int skip_prompts, const int32_t* outs, int spec, int T,
                                  int64_t num_blocks, void* stream) {
     // G = 4 runs the decode records, other groups the verify records
-    const bool vrec = Hkv > 0 && Hq != 4 * Hkv;
+    const int G = Hkv > 0 && Hq % Hkv == 0 ? Hq / Hkv : 0;
+    const int nr = Hkv <= 0 || G == 4 ? 1 : G > 0 ? pkv::vf_rows(G) : pkv::VF_ROWS;
     if (T < 0 || Hq <= 0 ||
-        decode_layout(T, Hq, decode_n_wg(), vrec, Hkv > 0 && Hq % Hkv == 0 ? Hq / Hkv : 0).total >
+        decode_layout(T, Hq, decode_n_wg(), nr).total >
             PKV_NOALLOC_SCRATCH_BYTES) {
         t_fp8 = {nullptr, nullptr, 0, 0};  // the failed call still consumes a pending FP8 request
         return T < 0 || Hq <= 0 ? PKV_ERR_INVALID : PKV_ERR_UNSUPPORTED;

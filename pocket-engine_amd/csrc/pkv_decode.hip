@@ -569,13 +569,14 @@ struct StepAppend {
 // t: lenf(t)), cut into at most p.n_wg equal ranges of R >= max(min_range,
 // ceil(W / n_wg)) keys, and the token t0 holding key `start` at offset off0.
 // The first workgroup also writes offs[t] (exclusive offsets), offs[T] = W
-// and offs[T + 1] = R for the merge. For T <= block size one scan serves
+// and offs[T + 1] = R (| rflag) for the merge. For T <= block size one scan serves
 // both; otherwise a first pass totals W and a second finds the offsets.
 // Called by the whole workgroup; returns false for a wave (or the whole
 // workgroup) whose range is empty. sh_t0: 2 ints per range of the workgroup.
 template <bool MULTI, class LenF>
 __device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWave<MULTI>& rw, LenF lenf, int* sh_scan,
-                                           int* sh_t0, int& start, int& end, int& t0, int& off0) {
+                                           int* sh_t0, int& start, int& end, int& t0, int& off0,
+                                           int rflag = 0) {
     const int T = p.T, nthr = blockDim.x, tid = threadIdx.x, b = blockIdx.x;
     const bool writer = b == 0 && blockIdx.y == 0;
     const bool one = T <= nthr;
@@ -606,7 +607,7 @@ __device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWav
     end = MULTI ? min(W, start + min(W, R)) : min(W, start + R);
     if (writer && tid == 0) {
         p.offs[T] = W;
-        p.offs[T + 1] = R;
+        p.offs[T + 1] = R | rflag;
     }
     // token t at `off` with L keys: the workgroup's ranges that start in it
     auto mark = [&](int t, int off, int L) {

@@ -62,8 +62,46 @@ __device__ __forceinline__ int seg_len(int t, int T, const int* __restrict__ pos
     return L;
 }
 
-// One wave: segment headed by token t (rows t + r, r < vf_rows(G),
-// attending Lr[r] keys; Lr = 0 for absent rows), kv head kvh with G query
+// What the verify kernels walk, in LDS for up to MAX tokens: per token its
+// attended keys, position, sequence, its row in the sequence and the rows left
+// from it on. Filled by the whole workgroup in two dependent round trips;
+// without it every segment met costs the chain tok_seq -> cu -> pos again (24
+// query heads, 1 sequence of 500 keys 14.9 -> 14.5 us, 200 of 40 to 2,500
+// 134.6 -> 133.5, 48 x 4 draft rows at 16 heads over 2,000 keys 26.0 -> 25.0).
+struct SegTable {
+    static constexpr int MAX = 256;
+    int len[MAX], pos[MAX], seq[MAX], rel[MAX], left[MAX];
+    __device__ __forceinline__ void fill(const DecodeParams& p, const int* __restrict__ pos_,
+                                         const int* __restrict__ tok_seq, const int* __restrict__ cu,
+                                         const int* __restrict__ outs) {
+        for (int t = threadIdx.x; t < p.T; t += blockDim.x) {
+            const int s = tok_seq[t], x = pos_[t];
+            const int c0 = cu[s], c1 = cu[s + 1];
+            const bool prompt = p.skip_prompts && c1 - c0 > 1 && !is_spec(outs, p.spec, s);
+            len[t] = prompt ? 0 : x + 1;
+            pos[t] = x;
+            seq[t] = s;
+            rel[t] = t - c0;
+            left[t] = min(c1, p.T) - t;
+        }
+        __syncthreads();
+    }
+    // Keys of the segment of nr rows headed by t, as seg_len.
+    __device__ __forceinline__ int seg_len(int nr, int t, int& nrows) const {
+        nrows = rel[t] & (nr - 1) ? 0 : min(nr, left[t]);
+        int L = 0;
+        for (int r = 0; r < nrows; r++) L = max(L, len[t + r]);
+        return L;
+    }
+};
+
+// Two-block kernels: keys per range under which segments hold half the rows
+// (walk_segments), and the flag in offs[T + 1] that tells the merge.
+constexpr int SEG_HALF_KEYS = 96;
+constexpr int SEG_HALF_FLAG = 1 << 30;
+
+// One wave: segment headed by token t (rows t + r, r < NR, attending Lr[r]
+// keys; Lr = 0 for absent rows), kv head kvh with G query
 // heads, keys [j0, j1), bf16 cache (an E4M3 cache runs piece_body8,
 // pkv_decode8.hip). MFMA column c is row c / G, head c % G.
 // The result goes to epi(r, g, gq, acc, m, l) on the lanes of attending rows:
@@ -75,28 +113,41 @@ __device__ __forceinline__ int seg_len(int t, int T, const int* __restrict__ pos
 // row0 + position - P0 of k_rows / v_rows) instead of the cache, chosen per
 // lane on the pages that hold such keys (from the page of P0 on); earlier
 // pages take the plain cache addresses.
-template <int G, bool FUSED = false, class Epi>
+template <int G, bool FUSED = false, int NR = vf_rows(G), class Epi>
 __device__ __forceinline__ void verify_piece(const DecodeParams& p, const int* __restrict__ bt, uint16_t* vl, int t,
                                              int kvh, int j0, int j1, const int (&Lr)[VF_ROWS], Epi epi,
                                              int P0 = INT_MAX, int row0 = 0) {
-    constexpr int NR = vf_rows(G);
+    // Column blocks: RB rows each
+    constexpr int NB = NR * G > 16 ? 2 : 1, RB = NR / NB;
+    static_assert(RB * G <= 16, "16 columns hold a block's rows x heads");
     const int lane = threadIdx.x & 63, c16 = lane & 15, gq = lane >> 4;
     const int r_me = c16 / G, g_me = c16 % G;
-    const int myL = r_me >= NR ? 0 : r_me == 0 ? Lr[0] : r_me == 1 ? Lr[1] : r_me == 2 ? Lr[2] : Lr[3];
+    const int L0 = Lr[0], L1 = Lr[1], L2 = Lr[2], L3 = Lr[3];
+    int myL[NB];
+    if constexpr (NB == 1) {
+        myL[0] = r_me >= RB ? 0 : r_me == 0 ? L0 : r_me == 1 ? L1 : r_me == 2 ? L2 : L3;
+    } else {
+        static_assert(NB == 1 || RB == 2, "two blocks of two rows");
+        myL[0] = r_me == 0 ? L0 : r_me == 1 ? L1 : 0;
+        myL[1] = r_me == 0 ? L2 : r_me == 1 ? L3 : 0;
+    }
     const float sl2 = p.scale * LOG2E;
     const size_t row_elems = (size_t)p.Hkv * HEAD_DIM;  // slot row, elements
 
     // q.k over the 256 dims in 8 steps of 32: step c, lane group gq takes
     // dims dim0(c) .. + 7 (the same for q and k).
     auto dim0 = [&](int c) { return 32 * c + 8 * gq; };
-    bf16x8 qf[8];
-    if (myL > 0) {
-        const uint16_t* qrow = p.q + ((size_t)(t + r_me) * p.Hq + kvh * G + g_me) * HEAD_DIM;
+    bf16x8 qf[NB][8];
 #pragma unroll
-        for (int c = 0; c < 8; c++) qf[c] = as_bf16x8(*reinterpret_cast<const uint4*>(qrow + dim0(c)));
-    } else {
+    for (int n = 0; n < NB; n++) {
+        if (myL[n] > 0) {
+            const uint16_t* qrow = p.q + ((size_t)(t + n * RB + r_me) * p.Hq + kvh * G + g_me) * HEAD_DIM;
 #pragma unroll
-        for (int c = 0; c < 8; c++) qf[c] = as_bf16x8(make_uint4(0, 0, 0, 0));
+            for (int c = 0; c < 8; c++) qf[n][c] = as_bf16x8(*reinterpret_cast<const uint4*>(qrow + dim0(c)));
+        } else {
+#pragma unroll
+            for (int c = 0; c < 8; c++) qf[n][c] = as_bf16x8(make_uint4(0, 0, 0, 0));
+        }
     }
     auto page_of = [&](int pi) -> long {
         const long pg = bt[pi];
@@ -149,10 +200,15 @@ __device__ __forceinline__ void verify_piece(const DecodeParams& p, const int* _
         return as_bf16x8(B.kb[c]);
     };
 
-    f32x4 acc[16];
+    f32x4 acc[NB][16];
+    float m[NB], l[NB];
 #pragma unroll
-    for (int db = 0; db < 16; db++) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
+    for (int n = 0; n < NB; n++) {
+#pragma unroll
+        for (int db = 0; db < 16; db++) acc[n][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+        m[n] = -INFINITY;
+        l[n] = 0.f;
+    }
 
     // transposed-read address of this lane: key row 4 gq + c16 / 4, dims 4 (c16 % 4) + 16 db
     const uint16_t* tr = vl + (4 * gq + (c16 >> 2)) * VF_VSTR + 4 * (c16 & 3);
@@ -166,9 +222,14 @@ __device__ __forceinline__ void verify_piece(const DecodeParams& p, const int* _
     struct NONE {};
     auto page = [&](Buf& B, int pi, int nxt, auto prefetch) {
         constexpr bool PREFETCH = !std::is_same_v<decltype(prefetch), NONE>;
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        f32x4 s[NB];
 #pragma unroll
-        for (int c = 0; c < 8; c++) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k_frag(B, c), qf[c], s, 0, 0, 0);
+        for (int n = 0; n < NB; n++) s[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 8; c++)
+#pragma unroll
+            for (int n = 0; n < NB; n++)
+                s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k_frag(B, c), qf[n][c], s[n], 0, 0, 0);
         // rows of keys outside [j0, j1) as zeros: their weight is 0, and
         // a stale slot may hold NaN
 #pragma unroll
@@ -183,42 +244,49 @@ __device__ __forceinline__ void verify_piece(const DecodeParams& p, const int* _
             load_v(B, next, nxt, prefetch);
         }
         const int k0 = pi * PAGE + 4 * gq;
-        float sc[4], mx = -INFINITY;
+        s16x4 pb_hi[NB], pb_lo[NB];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int kp = k0 + i;
-            sc[i] = (kp >= j0 && kp < j1 && kp < myL) ? s[i] * sl2 : -INFINITY;
-            mx = fmaxf(mx, sc[i]);
+        for (int n = 0; n < NB; n++) {
+            float sc[4], mx = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int kp = k0 + i;
+                sc[i] = (kp >= j0 && kp < j1 && kp < myL[n]) ? s[n][i] * sl2 : -INFINITY;
+                mx = fmaxf(mx, sc[i]);
+            }
+            mx = max_xor32(max_xor16(mx));
+            const float mn = fmaxf(m[n], mx);
+            const float mref = mn == -INFINITY ? 0.f : mn;  // a column with no key yet keeps zeros
+            const float corr = __builtin_amdgcn_exp2f(m[n] - mref);
+            float pr[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) pr[i] = __builtin_amdgcn_exp2f(sc[i] - mref);
+            // P^T as a bf16 high part plus a bf16 remainder (two MFMAs, ~16
+            // mantissa bits): decode rows keep their weights in f32 (the
+            // reference's attn_paged_g4), which one bf16 per weight would miss by
+            // up to 2^-9 relative; the denominator sums the f32 weights.
+            const uint32_t h01 = pack2_hw(pr[0], pr[1]), h23 = pack2_hw(pr[2], pr[3]);
+            const uint32_t r01 = pack2_hw(pr[0] - bf_lo(h01), pr[1] - bf_hi(h01));
+            const uint32_t r23 = pack2_hw(pr[2] - bf_lo(h23), pr[3] - bf_hi(h23));
+            l[n] = l[n] * corr + ((pr[0] + pr[1]) + (pr[2] + pr[3]));
+            m[n] = mn;
+            if (__any(corr != 1.f)) {
+#pragma unroll
+                for (int db = 0; db < 16; db++) acc[n][db] *= corr;
+            }
+            pb_hi[n] = __builtin_bit_cast(s16x4, make_uint2(h01, h23));
+            pb_lo[n] = __builtin_bit_cast(s16x4, make_uint2(r01, r23));
         }
-        mx = max_xor32(max_xor16(mx));
-        const float mn = fmaxf(m, mx);
-        const float mref = mn == -INFINITY ? 0.f : mn;  // a column with no key yet keeps zeros
-        const float corr = __builtin_amdgcn_exp2f(m - mref);
-        float pr[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) pr[i] = __builtin_amdgcn_exp2f(sc[i] - mref);
-        // P^T as a bf16 high part plus a bf16 remainder (two MFMAs, ~16
-        // mantissa bits): decode rows keep their weights in f32 (the
-        // reference's attn_paged_g4), which one bf16 per weight would miss by
-        // up to 2^-9 relative; the denominator sums the f32 weights.
-        const uint32_t h01 = pack2_hw(pr[0], pr[1]), h23 = pack2_hw(pr[2], pr[3]);
-        const uint32_t r01 = pack2_hw(pr[0] - bf_lo(h01), pr[1] - bf_hi(h01));
-        const uint32_t r23 = pack2_hw(pr[2] - bf_lo(h23), pr[3] - bf_hi(h23));
-        l = l * corr + ((pr[0] + pr[1]) + (pr[2] + pr[3]));
-        m = mn;
-        if (__any(corr != 1.f)) {
-#pragma unroll
-            for (int db = 0; db < 16; db++) acc[db] *= corr;
-        }
-        const s16x4 pb_hi = __builtin_bit_cast(s16x4, make_uint2(h01, h23));
-        const s16x4 pb_lo = __builtin_bit_cast(s16x4, make_uint2(r01, r23));
         wave_sync();  // V staged
 #pragma unroll
         for (int db = 0; db < 16; db++) {
             const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                 (__attribute__((address_space(3))) s16x4*)(tr + 16 * db));
-            acc[db] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, pb_hi, acc[db], 0, 0, 0);
-            acc[db] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, pb_lo, acc[db], 0, 0, 0);
+#pragma unroll
+            for (int n = 0; n < NB; n++) {
+                acc[n][db] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, pb_hi[n], acc[n][db], 0, 0, 0);
+                acc[n][db] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, pb_lo[n], acc[n][db], 0, 0, 0);
+            }
         }
         wave_sync();  // reads done before the next page is staged
     };
@@ -244,15 +312,17 @@ __device__ __forceinline__ void verify_piece(const DecodeParams& p, const int* _
     }
     page(A, pg1, 0, NONE{});
 
-    l = add_xor32(add_xor16(l));
-    if (myL == 0) return;
-    epi(r_me, g_me, gq, acc, m, l);
+#pragma unroll
+    for (int n = 0; n < NB; n++) {
+        const float sum = add_xor32(add_xor16(l[n]));
+        if (myL[n] > 0) epi(n * RB + r_me, g_me, gq, acc[n], m[n], sum);
+    }
 }
 
 // Writes a verify piece's result for the lanes of (row r, head g): the gated
 // output when the piece holds all of the segment's keys, else the partial
-// record at index idx (vf_rows(G) records per index, one per segment row).
-template <int G>
+// record at index idx (NR records per index, one per segment row).
+template <int G, int NR = vf_rows(G)>
 struct VerifyEpi {
     const DecodeParams& p;
     int t, kvh, idx;
@@ -270,7 +340,7 @@ struct VerifyEpi {
                     gate4(acc[db][0], acc[db][1], acc[db][2], acc[db][3], inv, graw);
             }
         } else {
-            const size_t row = ((size_t)idx * vf_rows(G) + r) * p.Hq + h;
+            const size_t row = ((size_t)idx * NR + r) * p.Hq + h;
             float* pa = p.part_acc + row * HEAD_DIM + 4 * gq;
 #pragma unroll
             for (int db = 0; db < 16; db++)
@@ -280,65 +350,117 @@ struct VerifyEpi {
     }
 };
 
-// Key-range kernel over segments of vf_rows(G) rows; grid (n_wg,
-// ceil(Hkv / 4)), 64 * min(Hkv, 4) threads. Same range split as
-// decode_range_kernel with segment lengths in place of token lengths; block 0
-// writes offs[t] (segment offsets by head token, equal neighbours for other
-// tokens), offs[T] = W, offs[T + 1] = R. The bound caps it at 256 VGPRs (no
-// spills); it runs one workgroup per CU (two ranges per CU measured slower:
-// 856 against 817 us at C5).
+// The wave's range of the segments' keys, then each of its segment pieces to
+// piece(t, nr, Lr, seq, row0, P0, j0, j1, direct): the segment headed by t (nr
+// rows, row r attending Lr[r] keys, of sequence seq whose first row is row0 at
+// position P0), keys [j0, j1) of the sequence, and whether they are all of the
+// segment's. before() runs between the search's loads and its end. HALVES (two
+// column blocks): a short step, under SEG_HALF_KEYS keys a range, takes NR / 2
+// rows to a segment: more and shorter segments, each of one block.
+template <int NR, bool HALVES, bool MULTI, class Before, class Piece>
+__device__ __forceinline__ void walk_segments(const DecodeParams& p, const RangeWave<MULTI>& rw, SegTable& tab,
+                                              int* sh_scan, int* sh_t0, const int* __restrict__ pos,
+                                              const int* __restrict__ tok_seq, const int* __restrict__ cu,
+                                              const int* __restrict__ outs, Before before, Piece piece) {
+    const int T = p.T;
+    const bool tabled = T <= SegTable::MAX;
+    if (tabled) tab.fill(p, pos, tok_seq, cu, outs);
+    int nr, start, end, t0, off0;
+    // rows per segment: NR, or NR / 2
+    int nrs = NR;
+    if constexpr (HALVES) {
+        if (tabled) {
+            int W;
+            for (int base = 0, run = W = 0; base < T; base += blockDim.x) {
+                const int t = base + threadIdx.x;
+                block_scan(t < T ? tab.seg_len(NR, t, nr) : 0, sh_scan, run);
+                W += run;
+            }
+            if (__builtin_amdgcn_readfirstlane(W) < SEG_HALF_KEYS * p.n_wg) nrs = NR / 2;
+        }
+    }
+    auto len_at = [&](int t) {
+        return tabled ? tab.seg_len(nrs, t, nr) : seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr);
+    };
+    const bool any = find_range(p, rw, len_at, sh_scan, sh_t0, start, end, t0, off0,
+                                nrs < NR ? SEG_HALF_FLAG : 0);
+    before();
+    if (!any) return;
+    int t = t0, off = off0;
+    while (off < end && t < T) {
+        const int Ls = __builtin_amdgcn_readfirstlane(len_at(t));
+        nr = __builtin_amdgcn_readfirstlane(nr);
+        if (Ls > 0) {
+            int Lr[VF_ROWS], seq, row0, P0;
+            if (tabled) {
+#pragma unroll
+                for (int r = 0; r < VF_ROWS; r++)
+                    Lr[r] = r < nr ? __builtin_amdgcn_readfirstlane(tab.len[t + r]) : 0;
+                seq = __builtin_amdgcn_readfirstlane(tab.seq[t]);
+                row0 = t - __builtin_amdgcn_readfirstlane(tab.rel[t]);
+                P0 = __builtin_amdgcn_readfirstlane(tab.pos[row0]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < VF_ROWS; r++)
+                    Lr[r] = r < nr ? __builtin_amdgcn_readfirstlane(
+                                         decode_len(t + r, pos, tok_seq, cu, p.skip_prompts, outs, p.spec))
+                                   : 0;
+                seq = __builtin_amdgcn_readfirstlane(tok_seq[t]);
+                row0 = __builtin_amdgcn_readfirstlane(cu[seq]);
+                P0 = __builtin_amdgcn_readfirstlane(pos[row0]);
+            }
+            const int j0 = max(start, off) - off, j1 = min(end, off + Ls) - off;
+            piece(t, nr, Lr, seq, row0, P0, j0, j1, j0 == 0 && j1 == Ls && !p.fo.mode);
+            off += Ls;
+        }
+        t += max(nr, 1);  // the next segment's head (nr = 0: t heads none)
+    }
+}
+
+// Key-range kernel over segments of NR rows; grid (workgroups,
+// ceil(Hkv / 4)), 64 * min(Hkv, 4) threads (MULTI: 256, RangeWave). Same range
+// split as decode_range_kernel with segment lengths in place of token lengths;
+// block 0 writes offs[t] (segment offsets by head token, equal neighbours for
+// other tokens), offs[T] = W, offs[T + 1] = R. One column block: the bound caps
+// it at 256 VGPRs (no spills); it runs one workgroup per CU (two ranges per CU
+// measured slower: 856 against 817 us at C5).
+// NR x G > 16 (draft rows of 6 or 8 heads per kv head): two column blocks of
+// NR / 2 rows share every K and V^T fragment, so 4 rows read their pages once
+// instead of twice: 24 sequences x 4 rows at 24 query heads, 900 to
+// 16,000 keys, 188 -> 107 us;
+// 8 of 20,000 to 60,000 371 -> 209 with the merge. A segment of up to NR / 2 rows takes the
+// one-block body.
 // FUSED (the fused decode step for groups other than 4): the kernel also
 // appends the step's K/V rows (StepAppend) and reads the keys the step feeds
 // from those source rows (verify_piece), so no range waits for a write.
-template <int G, bool FUSED, bool MULTI>
-__global__ void __launch_bounds__(256, 2)
+template <int G, int NR, bool FUSED, bool MULTI>
+__global__ void __launch_bounds__(256, NR * G > 16 ? 1 : 2)
     verify_range_kernel(DecodeParams p, const int* __restrict__ pos, const int* __restrict__ tok_seq,
                         const int* __restrict__ block_table, const int* __restrict__ cu,
                         const int* __restrict__ outs, const int* __restrict__ slot_map) {
-    constexpr int NR = vf_rows(G);
     __shared__ int sh_scan[16];
     __shared__ int sh_t0[8];
+    __shared__ SegTable sh_tab;
     __shared__ __align__(16) uint16_t sh_v[4][VF_LDS];
-    const int T = p.T;
     const RangeWave<MULTI> rw(p);
-    const int b = rw.b;
     StepAppend<MULTI> app(rw);
     if constexpr (FUSED) app.begin(p, slot_map);
-    int nr, start, end, t0, off0;
-    const bool any = find_range(
-        p, rw, [&](int t) { return seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr); }, sh_scan,
-        sh_t0, start, end, t0, off0);
-    if constexpr (FUSED) app.finish(p, slot_map);
-    if (!any) return;
-    const int wave = rw.wave, kvh = rw.kvh;
-    int t = t0, off = off0;
-    while (off < end && t < T) {
-        const int Ls =
-            __builtin_amdgcn_readfirstlane(seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr));
-        if (Ls > 0) {
-            nr = __builtin_amdgcn_readfirstlane(nr);
-            int Lr[VF_ROWS];
-#pragma unroll
-            for (int r = 0; r < VF_ROWS; r++)
-                Lr[r] = r < nr ? __builtin_amdgcn_readfirstlane(
-                                     decode_len(t + r, pos, tok_seq, cu, p.skip_prompts, outs, p.spec))
-                               : 0;
-            const int seq = __builtin_amdgcn_readfirstlane(tok_seq[t]);
-            const int j0 = max(start, off) - off, j1 = min(end, off + Ls) - off;
-            const VerifyEpi<G> epi{p, t, kvh, t + b, j0 == 0 && j1 == Ls && !p.fo.mode};
-            if constexpr (FUSED) {
-                // the sequence's first row this step and its position
-                const int row0 = __builtin_amdgcn_readfirstlane(cu[seq]);
-                const int P0 = __builtin_amdgcn_readfirstlane(pos[row0]);
-                verify_piece<G, true>(p, block_table + (size_t)seq * p.max_blocks, sh_v[wave], t, kvh, j0, j1, Lr,
-                                      epi, P0, row0);
-            } else {
-                verify_piece<G>(p, block_table + (size_t)seq * p.max_blocks, sh_v[wave], t, kvh, j0, j1, Lr, epi);
+    walk_segments<NR, (NR * G > 16)>(
+        p, rw, sh_tab, sh_scan, sh_t0, pos, tok_seq, cu, outs,
+        [&]() {
+            if constexpr (FUSED) app.finish(p, slot_map);
+        },
+        [&](int t, int nr, const int(&Lr)[VF_ROWS], int seq, int row0, int P0, int j0, int j1, bool direct) {
+            const int* bt = block_table + (size_t)seq * p.max_blocks;
+            const VerifyEpi<G, NR> epi{p, t, rw.kvh, t + rw.b, direct};
+            if constexpr (NR * G > 16) {
+                if (nr <= NR / 2) {
+                    verify_piece<G, FUSED, NR / 2>(p, bt, sh_v[rw.wave], t, rw.kvh, j0, j1, Lr, epi, P0, row0);
+                    return;
+                }
             }
-            off += Ls;
-        }
-        t++;
-    }
+            verify_piece<G, FUSED, NR>(p, bt, sh_v[rw.wave], t, rw.kvh, j0, j1, Lr, epi, P0, row0);
+        });
 }
 
 // The same over an E4M3 cache with the E4M3 decode body (two pages per
@@ -352,44 +474,25 @@ __global__ void __launch_bounds__(256, 2)
     constexpr int NR = vf_rows(G);
     __shared__ int sh_scan[16];
     __shared__ int sh_t0[8];
+    __shared__ SegTable sh_tab;
     __shared__ WaveLds8 sh_w8[4];
-    const int T = p.T;
     const RangeWave<MULTI> rw(p);
-    const int b = rw.b;
-    int nr, start, end, t0, off0;
-    if (!find_range(
-            p, rw, [&](int t) { return seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr); }, sh_scan,
-            sh_t0, start, end, t0, off0))
-        return;
-    const int wave = rw.wave, kvh = rw.kvh;
-    int t = t0, off = off0;
-    while (off < end && t < T) {
-        const int Ls =
-            __builtin_amdgcn_readfirstlane(seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr));
-        if (Ls > 0) {
-            nr = __builtin_amdgcn_readfirstlane(nr);
-            int Lr[VF_ROWS];
-#pragma unroll
-            for (int r = 0; r < VF_ROWS; r++)
-                Lr[r] = r < nr ? __builtin_amdgcn_readfirstlane(
-                                     decode_len(t + r, pos, tok_seq, cu, p.skip_prompts, outs, p.spec))
-                               : 0;
-            const int seq = __builtin_amdgcn_readfirstlane(tok_seq[t]);
-            const int j0 = max(start, off) - off, j1 = min(end, off + Ls) - off;
-            const VerifyEpi<G> vepi{p, t, kvh, t + b, j0 == 0 && j1 == Ls && !p.fo.mode};
+    walk_segments<NR, false>(
+        p, rw, sh_tab, sh_scan, sh_t0, pos, tok_seq, cu, outs, []() {},
+        [&](int t, int nr, const int(&Lr)[VF_ROWS], int seq, int row0, int P0, int j0, int j1, bool direct) {
+            const VerifyEpi<G> vepi{p, t, rw.kvh, t + rw.b, direct};
             auto epi = [&](int c, int gq, const f32x4 (&acc)[16], float m, float l) {
                 vepi(c / G, c % G, gq, acc, m, l);
             };
-            piece_body8<NR, G>(p, block_table + (size_t)seq * p.max_blocks, sh_w8[wave], t, kvh, j0, j1, epi, Lr);
-            off += Ls;
-        }
-        t++;
-    }
+            piece_body8<NR, G>(p, block_table + (size_t)seq * p.max_blocks, sh_w8[rw.wave], t, rw.kvh, j0, j1, epi,
+                               Lr);
+        });
 }
 
 // Merges the split segments: one block of 64 NW threads per (row, query
-// head) (NW as decode_merge_kernel's); row t's segment (NR rows) is headed
-// by the row at offset NR * floor((t - cu[s]) / NR) of its sequence.
+// head) (NW as decode_merge_kernel's); row t's segment (NR rows, or NR / 2 by
+// the range kernel's flag) is headed by the row at offset
+// NR * floor((t - cu[s]) / NR) of its sequence.
 template <int NR, int NW = 4>
 __global__ void __launch_bounds__(64 * NW)
     verify_merge_kernel(DecodeParams p, const int* __restrict__ pos, const int* __restrict__ tok_seq,
@@ -397,11 +500,11 @@ __global__ void __launch_bounds__(64 * NW)
     const int t = blockIdx.x, T = p.T;
     if (decode_len(t, pos, tok_seq, cu, p.skip_prompts, outs, p.spec) <= 0) return;
     const int c0 = cu[tok_seq[t]];
-    const int r = (t - c0) & (NR - 1), th = t - r;
+    const int rf = p.offs[T + 1], R = rf & ~SEG_HALF_FLAG, nrs = rf & SEG_HALF_FLAG ? NR / 2 : NR;
+    const int r = (t - c0) & (nrs - 1), th = t - r;
     if (th < 0) return;
     const int o0 = p.offs[th], o1 = p.offs[th + 1];
     if (o1 <= o0) return;
-    const int R = p.offs[T + 1];
     const int b0 = o0 / R, b1 = (o1 - 1) / R;
     if (b0 == b1 && !p.fo.mode) return;
     merge_head<NW>(p, t, (th + b0) * NR + r, NR, b1 - b0 + 1, blockIdx.y);
