@@ -285,12 +285,16 @@ struct DecodeEpi8 {
             const float inv = 1.f / l;
             const uint16_t* gate = p.qkv + (size_t)t * p.qstride + (size_t)h * 2 * HEAD_DIM + HEAD_DIM + 4 * gq;
             uint16_t* o = p.out + ((size_t)t * p.Hq + h) * HEAD_DIM + 4 * gq;
+            // all gates requested first: a load after a store (out and qkv may
+            // overlap for all that the compiler knows) waits a round trip of
+            // its own
+            uint2 graw[16];
 #pragma unroll
-            for (int db = 0; db < 16; db++) {
-                const uint2 graw = *reinterpret_cast<const uint2*>(gate + 16 * db);
+            for (int db = 0; db < 16; db++) graw[db] = *reinterpret_cast<const uint2*>(gate + 16 * db);
+#pragma unroll
+            for (int db = 0; db < 16; db++)
                 *reinterpret_cast<uint2*>(o + 16 * db) =
-                    gate4(acc[db][0], acc[db][1], acc[db][2], acc[db][3], inv, graw);
-            }
+                    gate4(acc[db][0], acc[db][1], acc[db][2], acc[db][3], inv, graw[db]);
         } else {
             const size_t row = (size_t)idx * p.Hq + h;
             float* pa = p.part_acc + row * HEAD_DIM + 4 * gq;

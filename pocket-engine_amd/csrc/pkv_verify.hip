@@ -333,12 +333,16 @@ struct VerifyEpi {
             const float inv = 1.f / l;
             const uint16_t* gate = p.qkv + (size_t)row_t * p.qstride + (size_t)h * 2 * HEAD_DIM + HEAD_DIM + 4 * gq;
             uint16_t* o = p.out + ((size_t)row_t * p.Hq + h) * HEAD_DIM + 4 * gq;
+            // all gates requested first: a load after a store (out and qkv may
+            // overlap for all that the compiler knows) waits a round trip of
+            // its own
+            uint2 graw[16];
 #pragma unroll
-            for (int db = 0; db < 16; db++) {
-                const uint2 graw = *reinterpret_cast<const uint2*>(gate + 16 * db);
+            for (int db = 0; db < 16; db++) graw[db] = *reinterpret_cast<const uint2*>(gate + 16 * db);
+#pragma unroll
+            for (int db = 0; db < 16; db++)
                 *reinterpret_cast<uint2*>(o + 16 * db) =
-                    gate4(acc[db][0], acc[db][1], acc[db][2], acc[db][3], inv, graw);
-            }
+                    gate4(acc[db][0], acc[db][1], acc[db][2], acc[db][3], inv, graw[db]);
         } else {
             const size_t row = ((size_t)idx * NR + r) * p.Hq + h;
             float* pa = p.part_acc + row * HEAD_DIM + 4 * gq;
@@ -426,10 +430,9 @@ __device__ __forceinline__ void walk_segments(const DecodeParams& p, const Range
 // measured slower: 856 against 817 us at C5).
 // NR x G > 16 (draft rows of 6 or 8 heads per kv head): two column blocks of
 // NR / 2 rows share every K and V^T fragment, so 4 rows read their pages once
-// instead of twice: 24 sequences x 4 rows at 24 query heads, 900 to
-// 16,000 keys, 188 -> 107 us;
-// 8 of 20,000 to 60,000 371 -> 209 with the merge. A segment of up to NR / 2 rows takes the
-// one-block body.
+// instead of twice: 24 sequences x 4 rows at 24 query heads, 900 to 16,000
+// keys, 188 -> 107 us; 8 of 20,000 to 60,000, with the merge, 371 -> 209. A
+// segment of up to NR / 2 rows takes the one-block body.
 // FUSED (the fused decode step for groups other than 4): the kernel also
 // appends the step's K/V rows (StepAppend) and reads the keys the step feeds
 // from those source rows (verify_piece), so no range waits for a write.
