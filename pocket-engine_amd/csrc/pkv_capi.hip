@@ -642,31 +642,39 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
         const int st = launch_status();
         if (st != PKV_OK) return st;
     }
-    if ((phases & 2) && verify) {
-        // waves per (row, head) block chosen as for decode_merge_kernel below
-        using MergeKernel = void (*)(pkv::DecodeParams, const int*, const int*, const int*, const int*);
-        const int nw = (int64_t)T * Hq < device_cus() ? 16 : (int64_t)T + n_wg <= 12 * (int64_t)T ? 1 : 4;
-        const bool r4 = nr == 4;
-        const MergeKernel mk = nw == 16 ? (r4 ? pkv::verify_merge_kernel<4, 16> : pkv::verify_merge_kernel<2, 16>)
-                               : nw == 1 ? (r4 ? pkv::verify_merge_kernel<4, 1> : pkv::verify_merge_kernel<2, 1>)
-                                         : (r4 ? pkv::verify_merge_kernel<4, 4> : pkv::verify_merge_kernel<2, 4>);
-        hipLaunchKernelGGL(mk, dim3(T, Hq), dim3(64 * nw), 0, (hipStream_t)stream, p, pos, tok_seq, cu, outs);
-        return launch_status();
-    }
     if (phases & 2) {
         // Waves per (token, head) block: 16 when there are fewer blocks than
-        // CUs (a head's records, up to one per range, load in one round);
-        // one when a token has at most 12 records on average ((T + n_wg) / T:
-        // one wave folds 16 per round and skips the cross-wave combine;
-        // measured faster at 9, the E4M3 C3 step's two ranges per CU, and
-        // slower at 17); else 4. Any count is correct; this only picks the
-        // faster launch.
-        if ((int64_t)T * Hq < device_cus())
-            hipLaunchKernelGGL(pkv::decode_merge_kernel<16>, dim3(T, Hq), dim3(1024), 0, (hipStream_t)stream, p);
-        else if ((int64_t)T + n_wg <= 12 * (int64_t)T)
-            hipLaunchKernelGGL(pkv::decode_merge_kernel<1>, dim3(T, Hq), dim3(64), 0, (hipStream_t)stream, p);
-        else
-            hipLaunchKernelGGL(pkv::decode_merge_kernel<4>, dim3(T, Hq), dim3(256), 0, (hipStream_t)stream, p);
+        // CUs (a head's records, up to one per range, load in one round), as
+        // 4 blocks of 64 dims while those still fit the CUs (the whole step of
+        // 1 sequence of 4,096 keys 15.1 -> 13.7 us, of 60,000 over E4M3 45.7 ->
+        // 40.1, 4 sequences 24.9 -> 24.2; with 128 such blocks 0.5 us slower,
+        // with 192 or more 3 to 10 %); one
+        // when a token has at most 12 records on average ((T + n_wg) / T: one
+        // wave folds 16 per round and skips the cross-wave combine; measured
+        // faster at 9, the E4M3 C3 step's two ranges per CU, and slower at
+        // 17); else 4. Any count is correct; this only picks the faster launch.
+        using MergeKernel = void (*)(pkv::DecodeParams);
+        using VerifyMergeKernel = void (*)(pkv::DecodeParams, const int*, const int*, const int*, const int*);
+        const int64_t blocks = (int64_t)T * Hq, cus = device_cus();
+        const int nw = 4 * blocks <= cus && !fo.mode ? 0
+                       : blocks < cus                ? 16
+                       : (int64_t)T + n_wg <= 12 * (int64_t)T ? 1 : 4;
+        const dim3 grid(T, Hq, nw == 0 ? 4 : 1), block(nw == 0 ? 1024 : 64 * nw);
+        if (verify) {
+            const bool r4 = nr == 4;
+            const VerifyMergeKernel mk =
+                nw == 0    ? (r4 ? pkv::verify_merge_kernel<4, 0> : pkv::verify_merge_kernel<2, 0>)
+                : nw == 16 ? (r4 ? pkv::verify_merge_kernel<4, 16> : pkv::verify_merge_kernel<2, 16>)
+                : nw == 1  ? (r4 ? pkv::verify_merge_kernel<4, 1> : pkv::verify_merge_kernel<2, 1>)
+                           : (r4 ? pkv::verify_merge_kernel<4, 4> : pkv::verify_merge_kernel<2, 4>);
+            hipLaunchKernelGGL(mk, grid, block, 0, (hipStream_t)stream, p, pos, tok_seq, cu, outs);
+        } else {
+            const MergeKernel mk = nw == 0    ? pkv::decode_merge_kernel<0>
+                                   : nw == 16 ? pkv::decode_merge_kernel<16>
+                                   : nw == 1  ? pkv::decode_merge_kernel<1>
+                                              : pkv::decode_merge_kernel<4>;
+            hipLaunchKernelGGL(mk, grid, block, 0, (hipStream_t)stream, p);
+        }
         return launch_status();
     }
     return PKV_OK;

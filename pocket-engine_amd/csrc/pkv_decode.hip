@@ -237,17 +237,106 @@ __device__ __forceinline__ void merge_rows(int n, float mscale, MsAt ms_at, AccA
     }
 }
 
+// The same for few (row, head) blocks of many records each, 64 of the head's
+// 256 dims per block (dims 64 part .. + 63): 16 lanes per record, 4 records to
+// a wave's load, 16 waves, so up to 256 records load in one round, from 4
+// times the CUs; the gate is requested with them. Bound by its dependent round
+// trips: 129 records x 16 heads took 5.6 us as one block a head, 1.4 us less
+// so. No FP8 copies (their groups span parts).
+template <class MsAt, class AccAt>
+__device__ __forceinline__ void merge_rows_part(int n, int part, MsAt ms_at, AccAt acc_at, const uint16_t* gate,
+                                                uint16_t* out) {
+    constexpr int NW = 16, U = 4;
+    __shared__ __align__(16) float sh_a[NW][64];
+    __shared__ float sh_ms[NW][2];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, rec = lane >> 4, d = 64 * part + 4 * (lane & 15);
+    const uint2 graw = *reinterpret_cast<const uint2*>(gate + d);
+    float M = -INFINITY, S = 0.f, A[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 4 * w + rec; i0 - rec < n; i0 += 4 * NW * U) {
+        float2 mu[U];
+        float2 lo[U], hi[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = i0 + 4 * NW * u;
+            mu[u] = make_float2(-INFINITY, 0.f);
+            lo[u] = hi[u] = make_float2(0.f, 0.f);
+            if (i < n) {
+                mu[u] = *reinterpret_cast<const float2*>(ms_at(i));
+                lo[u] = *reinterpret_cast<const float2*>(acc_at(i) + d);
+                hi[u] = *reinterpret_cast<const float2*>(acc_at(i) + d + 2);
+            }
+        }
+        float Mn = M;
+#pragma unroll
+        for (int u = 0; u < U; u++) Mn = fmaxf(Mn, mu[u].x);
+        const float ref = Mn == -INFINITY ? 0.f : Mn;  // nothing attended yet: every factor is 0
+        const float c = __builtin_amdgcn_exp2f(M - ref);
+        S *= c;
+#pragma unroll
+        for (int e = 0; e < 4; e++) A[e] *= c;
+        M = Mn;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const float f = __builtin_amdgcn_exp2f(mu[u].x - ref);
+            S += mu[u].y * f;
+            A[0] += lo[u].x * f;
+            A[1] += lo[u].y * f;
+            A[2] += hi[u].x * f;
+            A[3] += hi[u].y * f;
+        }
+    }
+    // the wave's 4 record groups, then the waves, through LDS
+    auto fold = [&]() {
+        const float Mt = max_xor32(max_xor16(M));
+        const float f = Mt == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mt);
+        M = Mt;
+        S = add_xor32(add_xor16(S * f));
+#pragma unroll
+        for (int e = 0; e < 4; e++) A[e] = add_xor32(add_xor16(A[e] * f));
+    };
+    fold();
+    if (lane < 16) *reinterpret_cast<float4*>(&sh_a[w][4 * lane]) = make_float4(A[0], A[1], A[2], A[3]);
+    if (lane == 0) {
+        sh_ms[w][0] = M;
+        sh_ms[w][1] = S;
+    }
+    __syncthreads();
+    if (w != 0) return;
+    M = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < NW / 4; k++) M = fmaxf(M, sh_ms[4 * k + rec][0]);
+    S = A[0] = A[1] = A[2] = A[3] = 0.f;
+#pragma unroll
+    for (int k = 0; k < NW / 4; k++) {
+        const int v = 4 * k + rec;
+        const float mk = sh_ms[v][0];
+        const float f = mk == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mk - M);
+        const float4 b = *reinterpret_cast<const float4*>(&sh_a[v][4 * (lane & 15)]);
+        S += sh_ms[v][1] * f;
+        A[0] += b.x * f;
+        A[1] += b.y * f;
+        A[2] += b.z * f;
+        A[3] += b.w * f;
+    }
+    fold();
+    if (lane < 16) *reinterpret_cast<uint2*>(out + d) = gate4(A[0], A[1], A[2], A[3], 1.f / S, graw);
+}
+
 // Merges this library's partials of token t, query head h: record i is row
-// (base + i * stride) * Hq + h of part_ms / part_acc.
+// (base + i * stride) * Hq + h of part_ms / part_acc. NW = 0: merge_rows_part
+// (blockIdx.z: the part).
 template <int NW = 4>
 __device__ __forceinline__ void merge_head(const DecodeParams& p, int t, int base, int stride, int n, int h) {
     const Fp8Out* fo = p.fo.mode ? &p.fo : nullptr;
     const size_t r0 = (size_t)base * p.Hq + h, step = (size_t)stride * p.Hq;
-    merge_rows<NW>(
-        n, 1.f, [&](int i) { return p.part_ms + (r0 + i * step) * 2; },
-        [&](int i) { return p.part_acc + (r0 + i * step) * HEAD_DIM; },
-        p.qkv + (size_t)t * p.qstride + (size_t)h * 2 * HEAD_DIM + HEAD_DIM, p.out + ((size_t)t * p.Hq + h) * HEAD_DIM,
-        fo, t, h * HEAD_DIM, p.Hq * HEAD_DIM);
+    auto ms_at = [&](int i) { return p.part_ms + (r0 + i * step) * 2; };
+    auto acc_at = [&](int i) { return p.part_acc + (r0 + i * step) * HEAD_DIM; };
+    const uint16_t* gate = p.qkv + (size_t)t * p.qstride + (size_t)h * 2 * HEAD_DIM + HEAD_DIM;
+    uint16_t* out = p.out + ((size_t)t * p.Hq + h) * HEAD_DIM;
+    if constexpr (NW == 0)
+        merge_rows_part(n, blockIdx.z, ms_at, acc_at, gate, out);
+    else
+        merge_rows<NW>(n, 1.f, ms_at, acc_at, gate, out, fo, t, h * HEAD_DIM, p.Hq * HEAD_DIM);
 }
 
 // One wave: token t, kv head kvh, keys [j0, j1) of its sequence. With FRESH,
@@ -728,9 +817,10 @@ __global__ void __launch_bounds__(256, 1)
 }
 
 // Combines the partials of tokens split over several ranges (after
-// decode_range_kernel). One block of 64 NW threads per (token, query head).
+// decode_range_kernel). One block of 64 NW threads per (token, query head), or
+// (NW = 0) 4 of 1,024.
 template <int NW>
-__global__ void __launch_bounds__(64 * NW) decode_merge_kernel(DecodeParams p) {
+__global__ void __launch_bounds__(NW ? 64 * NW : 1024) decode_merge_kernel(DecodeParams p) {
     const int t = blockIdx.x, T = p.T;
     const int o0 = p.offs[t], o1 = p.offs[t + 1];  // offs[T] = W
     if (o1 <= o0) return;
@@ -739,6 +829,7 @@ __global__ void __launch_bounds__(64 * NW) decode_merge_kernel(DecodeParams p) {
     if (b0 == b1 && !p.fo.mode) return;  // finished in place by its range
     merge_head<NW>(p, t, t + b0, 1, b1 - b0 + 1, blockIdx.y);
 }
+template __global__ void decode_merge_kernel<0>(DecodeParams);
 template __global__ void decode_merge_kernel<1>(DecodeParams);
 template __global__ void decode_merge_kernel<4>(DecodeParams);
 template __global__ void decode_merge_kernel<16>(DecodeParams);

@@ -497,7 +497,7 @@ __global__ void __launch_bounds__(256, 2)
 // the range kernel's flag) is headed by the row at offset
 // NR * floor((t - cu[s]) / NR) of its sequence.
 template <int NR, int NW = 4>
-__global__ void __launch_bounds__(64 * NW)
+__global__ void __launch_bounds__(NW ? 64 * NW : 1024)
     verify_merge_kernel(DecodeParams p, const int* __restrict__ pos, const int* __restrict__ tok_seq,
                         const int* __restrict__ cu, const int* __restrict__ outs) {
     const int t = blockIdx.x, T = p.T;
