@@ -60,9 +60,16 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return f2b_bits(
 // x / y for the gated epilogue (y = 1 + exp(-gate) >= 1): the reciprocal
 // and one residual correction (q + (x - y q) / y), which gives IEEE's
 // correctly rounded quotient except in rare last-bit cases, before the
-// bf16 rounding. An infinite x or y makes the residual NaN; q is then the
-// quotient (inf / y, x / inf = 0, inf / inf = NaN).
+// bf16 rounding; x / inf is 0 as in IEEE.
 __device__ __forceinline__ float gated_div(float x, float y) {
+    const float r = __builtin_amdgcn_rcpf(y), q = x * r;
+    const float c = __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
+    return __builtin_isinf(y) ? 0.f * x : c;
+}
+// The same for rows that may be infinite: an infinite x or y makes the
+// residual NaN; q is then the quotient (inf / y, x / inf = 0, inf / inf =
+// NaN). (In the prompt kernels' epilogue it cost 0.9 % of 4.2 ms.)
+__device__ __forceinline__ float gated_div_any(float x, float y) {
     const float r = __builtin_amdgcn_rcpf(y), q = x * r;
     const float c = __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
     return c == c ? c : q;
