@@ -198,13 +198,13 @@ int pkv_attn_decode_step_noalloc(const void* k_rows, const void* v_rows, int64_t
  * speculative rows (is_spec, src/kernels/qwen35.cu:94-100), which its
  * attn_paged_g<G> serves one token per block, each re-reading the
  * sequence's pages (launched at src/model.rs:2366-2437). Here up to 4
- * (G <= 4) or 2 (G = 6, 8) consecutive rows of a sequence share one pass
- * over its pages. `cu` is
+ * consecutive rows of a sequence share one pass over its pages. `cu` is
  * required and each sequence's rows must be consecutive (cu[s] ..
  * cu[s+1]-1, as Scheduler::fill writes them, src/sched.rs:1105-1115).
- * Segments hold 4 rows for G <= 4 and 2 rows for G = 6 or 8 (the 16 MFMA
- * columns are rows x query heads).
- * Workspace: pkv_attn_verify_workspace bytes. Shapes as pkv_attn_decode. */
+ * Segments hold 4 rows (G = 6 or 8: two blocks of 16 MFMA columns; 2 rows
+ * where a step has few keys, and over an E4M3 cache).
+ * Workspace: pkv_attn_verify_workspace bytes (G = 6 or 8 with a smaller one
+ * that holds 2 records per row: 2-row segments). Shapes as pkv_attn_decode. */
 int pkv_attn_verify_workspace(int T, int Hq, size_t* bytes);
 int pkv_attn_verify(const void* q, const void* kcache, const void* vcache, const void* qkv, int qstride, int Hq,
                     int Hkv, const int32_t* pos, const int32_t* tok_seq, const int32_t* block_table, int max_blocks,
