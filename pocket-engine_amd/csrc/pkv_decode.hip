@@ -113,19 +113,21 @@ struct WaveLds {
 };
 
 // Gated output of 4 dims: y = bf16(rbf(a * inv) * sigmoid(gate)) (reference
-// qwen35.cu:1290-1293), with the hardware's bf16 rounding and gated_div_any: 13
-// instructions a value where the software rounding and IEEE division took 45,
-// 64 values per lane when a verify or E4M3 piece finishes its row in place
-// (with the gates requested together, 200 sequences of 40 to 2,500 keys at 24
-// query heads 132 -> 118 us, 300 of 20 to 300 71.5 -> 60; over E4M3 at 16
-// heads 97 -> 79).
+// qwen35.cu:1290-1293), divided as IEEE has it (denormal quotients included)
+// and rounded by the hardware's bf16 conversion, in place of 2 x 5 instructions
+// of software rounding a value: 64 values per lane when a verify or E4M3 piece
+// finishes its row in place. With the gates requested together, 200 sequences
+// of 40 to 2,500 keys at 24 query heads 129.5 -> 117.0 us, 300 of 20 to 300
+// 71.3 -> 60.9; over E4M3 at 16 heads 100 -> 80.8. (The reciprocal and one
+// residual step, gated_div, saves another 1.5 us of the first, but gives 0 for
+// gates around -88 and is not always correctly rounded.)
 __device__ __forceinline__ uint2 gate4(float a0, float a1, float a2, float a3, float inv, uint2 graw,
                                        float* y = nullptr) {
     const uint32_t r01 = pack2_hw(a0 * inv, a1 * inv), r23 = pack2_hw(a2 * inv, a3 * inv);
-    const float y0 = gated_div_any(bf_lo(r01), 1.f + __expf(-bf_lo(graw.x)));
-    const float y1 = gated_div_any(bf_hi(r01), 1.f + __expf(-bf_hi(graw.x)));
-    const float y2 = gated_div_any(bf_lo(r23), 1.f + __expf(-bf_lo(graw.y)));
-    const float y3 = gated_div_any(bf_hi(r23), 1.f + __expf(-bf_hi(graw.y)));
+    const float y0 = bf_lo(r01) / (1.f + __expf(-bf_lo(graw.x)));
+    const float y1 = bf_hi(r01) / (1.f + __expf(-bf_hi(graw.x)));
+    const float y2 = bf_lo(r23) / (1.f + __expf(-bf_lo(graw.y)));
+    const float y3 = bf_hi(r23) / (1.f + __expf(-bf_hi(graw.y)));
     if (y) {
         y[0] = y0;
         y[1] = y1;
