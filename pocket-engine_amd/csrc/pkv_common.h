@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pkv_index.h"
+
 namespace pkv {
 
 constexpr int HEAD_DIM = 256;  // attention head width (reference model.rs:14)

@@ -698,15 +698,11 @@ __device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWav
     W = __builtin_amdgcn_readfirstlane(W);  // block-uniform: keep it in scalar registers
     int R = max(p.min_range, (W + p.n_wg - 1) / p.n_wg);
     if constexpr (MULTI) R = max(R, min(RANGE_KEYS, (W + p.nb - 1) / p.nb));
-    // MULTI: the workgroup's k-th range starts at key at(k) (W: past the last;
-    // n_wg R can pass the int range)
-    auto at = [&](int k) {
-        const unsigned long s = (unsigned long)(unsigned)(b + k * p.nb) * (unsigned)R;
-        return __builtin_amdgcn_readfirstlane(s < (unsigned long)W ? (int)s : W);
-    };
-    const int first = MULTI ? at(0) : b * R, last = MULTI ? at(rw.rpb - 1) : first;
+    // the workgroup's k-th range starts at key at(k) (W: past the last)
+    auto at = [&](int k) { return __builtin_amdgcn_readfirstlane(range_start(b + k * p.nb, R, W)); };
+    const int first = at(0), last = MULTI ? at(rw.rpb - 1) : first;
     start = MULTI ? at(rw.sub) : first;
-    end = MULTI ? min(W, start + min(W, R)) : min(W, start + R);
+    end = range_end(start, R, W);
     if (writer && tid == 0) {
         p.offs[T] = W;
         p.offs[T + 1] = R | rflag;

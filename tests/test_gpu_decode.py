@@ -139,6 +139,19 @@ def test_decode_split_configuration_invariance(dev, wg, mr):
     assert ok, err
 
 
+@pytest.mark.parametrize("T,Hkv", [(3, 4), (300, 2), (70, 1)])
+def test_decode_most_workgroups_and_longest_ranges(dev, T, Hkv):
+    """The largest settings that attn_decode_config takes: the starts of
+    ranges 2,048 to 16,383 (70 tokens at 1 kv head: 65,535) pass the 32-bit
+    range, and those ranges hold no key."""
+    print(f"case decode config wg=64 mr={1 << 20} T={T} Hkv={Hkv}", flush=True)
+    lens = [int(x) for x in np.random.default_rng(T).integers(1, 200, T)]
+    c = decode_case(lens, 4 * Hkv, Hkv, seed=T)
+    pkv.attn_decode_config(64, 1 << 20)
+    ok, err = close(run_gpu(c, dev, cu=c["cu"]), run_oracle(c))
+    assert ok, err
+
+
 def test_decode_c3_batch64_properties(dev):
     """Config 3 at full size (B = 64, contexts U[512, 8192], pages scattered
     over a 65,536-page pool): (1) moving every page to another place in the
