@@ -205,28 +205,20 @@ struct PrepLds {
     float c[ROPE_DIM / 2], s[ROPE_DIM / 2];
 };
 
-// One wave, token t: units u0 .. u0 + P - 1 of the row's Hq / 2 + 2 nk (nk =
-// ceil(Hkv / 2)) pairs of q, then k, then v heads; half-wave hv takes the
-// pair's head hv (an odd Hkv's last pair has one). Hq is even.
+// One wave, token t: units u0 .. u0 + P - 1 of the row's pairs of heads
+// (PrepPairs). A pair is of one kind, so whether it is stored (q always, k and
+// v with a slot) is one answer for the wave.
 template <int P>
 __device__ __forceinline__ void prep_units(const PrepArgs& a, PrepLds& lds, int t, int u0) {
     const int lane = threadIdx.x & 63, hv = lane >> 5, sub = lane & 31;
-    const int nq = a.Hq / 2, nk = (a.Hkv + 1) / 2, nu = nq + 2 * nk;
+    const PrepPairs pairs(a.Hq, a.Hkv);
+    const int nu = pairs.units();
     const uint16_t* row = a.qkv + (size_t)t * a.qstride;
     uint4 raw[P];
 #pragma unroll
     for (int i = 0; i < P; i++) {
-        // (past the last unit: the last one again, not stored; an absent
-        // head of a pair: head 0 of its kind)
-        const int u = min(u0 + i, nu - 1);
-        int src;  // in heads of 256
-        if (u < nq) {
-            src = 2 * (2 * u + hv);
-        } else {
-            const bool v = u >= nq + nk;
-            const int h = 2 * (u - nq - (v ? nk : 0)) + hv;
-            src = 2 * a.Hq + (v ? a.Hkv : 0) + (h < a.Hkv ? h : 0);
-        }
+        // (past the last unit: the last one again, not stored)
+        const int src = pairs.source(min(u0 + i, nu - 1), hv);  // in heads of 256
         const u32x4_a8 x = *reinterpret_cast<const u32x4_a8*>(row + (size_t)src * HEAD_DIM + 8 * sub);
         raw[i] = make_uint4(x.x, x.y, x.z, x.w);
     }
@@ -241,7 +233,7 @@ __device__ __forceinline__ void prep_units(const PrepArgs& a, PrepLds& lds, int 
         w[4] = w1.x, w[5] = w1.y, w[6] = w1.z, w[7] = w1.w;
     };
     float wq[8], wk[8];
-    norm8(P == 1 && u0 >= nq ? a.k_norm : a.q_norm, wq);
+    norm8(P == 1 && !pairs.is_q(u0) ? a.k_norm : a.q_norm, wq);
     if (P > 1) norm8(a.Hkv > 0 ? a.k_norm : a.q_norm, wk);
     {
         // cos / sin of d = sub
@@ -271,10 +263,10 @@ __device__ __forceinline__ void prep_units(const PrepArgs& a, PrepLds& lds, int 
     for (int i = 0; i < P; i++) {
         const int u = u0 + i;
         if (u >= nu) break;
-        const bool is_q = u < nq, is_v = u >= nq + nk;
+        const bool is_q = pairs.is_q(u), is_v = pairs.is_v(u);
         if (!is_q && !has_slot) break;  // (k and v units follow q's)
-        const int h = 2 * (u - (is_q ? 0 : is_v ? nq + nk : nq)) + hv;
-        const bool ok = is_q || h < a.Hkv;
+        const int h = pairs.head(u, hv);
+        const bool ok = pairs.has(u, hv);
         uint32_t y[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
         float x[8];
 #pragma unroll
