@@ -30,9 +30,10 @@ def t_(a, dev):
     return torch.from_numpy(a).to(dev)
 
 
-def test_prep_stores_e4m3(dev):
-    print("case prep e4m3", flush=True)
-    T, Hq, Hkv = 37, 16, 4
+# (odd head counts run the wave-per-head kernel)
+@pytest.mark.parametrize("T,Hq,Hkv", [(37, 16, 4), (29, 4, 1), (37, 3, 2), (20, 12, 3)])
+def test_prep_stores_e4m3(dev, T, Hq, Hkv):
+    print(f"case prep e4m3 T={T} Hq={Hq} Hkv={Hkv}", flush=True)
     c = prep_case(T, Hq, Hkv, 11, pool=64)
     pool = c["pool"]
     kc8 = np.full((pool, Hkv, D), 0x33, np.uint8)

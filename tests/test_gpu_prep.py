@@ -60,7 +60,8 @@ def check(c, qout, kc, vc, kc0, vc0):
         assert worst <= 1 and exact >= 0.99, f"{name}: max ulp {worst}, exact {exact:.4f}"
 
 
-@pytest.mark.parametrize("T,Hq,Hkv,seed", [(37, 16, 4, 0), (64, 8, 2, 1), (1, 4, 1, 2), (20, 24, 4, 3), (9, 32, 4, 4), (5, 2, 2, 5)])
+@pytest.mark.parametrize("T,Hq,Hkv,seed", [(37, 16, 4, 0), (64, 8, 2, 1), (1, 4, 1, 2), (20, 24, 4, 3), (9, 32, 4, 4), (5, 2, 2, 5),
+                                           (11, 3, 1, 6), (20, 5, 2, 7)])  # odd Hq: the wave-per-head kernel
 def test_prep_matches_oracle(dev, T, Hq, Hkv, seed):
     print(f"case prep T={T} Hq={Hq} Hkv={Hkv}", flush=True)
     c = case(T, Hq, Hkv, seed, pool=128)
@@ -134,6 +135,37 @@ def test_prep_many_rows_match_few(dev, T, Hq, Hkv, e4m3, pad):
         return o
 
     for name, a, b in zip(("q", "k", "v", "kscale", "vscale"), run(T), run(257)):
+        assert a is None or torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,e4m3", [(37, 16, 4, False), (1400, 16, 4, False), (1400, 16, 4, True),
+                                          (50, 24, 4, True), (41, 4, 1, False), (8200, 6, 1, False)])
+def test_paired_heads_match_wave_per_head(dev, T, Hq, Hkv, e4m3):
+    """pkv_attn_prep's paired heads (one and four pairs to a wave) give bit for
+    bit the code object's attn_prep, which takes a wave per head."""
+    print(f"case prep paired T={T} Hq={Hq} Hkv={Hkv} e4m3={e4m3}", flush=True)
+    c = case(T, Hq, Hkv, 13, pool=T + 5)
+    pool = c["pool"]
+    qkv = torch.from_numpy(c["qkv"].view(np.int16)).to(dev)
+    d = {k: torch.from_numpy(c[k]).to(dev) for k in ("q_norm", "k_norm", "rope", "slots", "inv_freq")}
+
+    def run(call):
+        cache = lambda: torch.full((pool, Hkv, D * (1 if e4m3 else 2)), 7, dtype=torch.uint8, device=dev)
+        scale = lambda: torch.full((pool, Hkv), -1.0, device=dev) if e4m3 else None
+        o = [torch.zeros(T, Hq, D, dtype=torch.int16, device=dev), cache(), cache(), scale(), scale()]
+        call(o)
+        torch.cuda.synchronize()
+        return o
+
+    paired = run(lambda o: pkv.attn_prep(qkv, c["qstride"], Hq, Hkv, d["q_norm"], d["k_norm"], d["rope"], T, 11, 11,
+                                         d["slots"], d["inv_freq"], o[0], o[1], o[2], 1e-6, T, pool, kscale=o[3],
+                                         vscale=o[4]))
+    rk = RefKernels()
+    single = run(lambda o: rk.launch("attn_prep", (T, Hq + 2 * Hkv, 1), 128, 0,
+                                     [P(qkv), I(c["qstride"]), I(Hq), I(Hkv), P(d["q_norm"]), P(d["k_norm"]),
+                                      P(d["rope"]), I(T), I(11), I(11), P(d["slots"]), P(d["inv_freq"]), P(o[0]),
+                                      P(o[1]), P(o[2]), P(o[3]), P(o[4]), F(1e-6)]))
+    for name, a, b in zip(("q", "k", "v", "kscale", "vscale"), paired, single):
         assert a is None or torch.equal(a, b), name
 
 
