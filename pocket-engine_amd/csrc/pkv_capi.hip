@@ -77,9 +77,23 @@ constexpr int F8_WG_PER_CU = 2;
 // head): this many times the ranges, as many to a workgroup (RangeWave<true>),
 // put 4 waves' bytes in flight again.
 int kv_head_ranges(int Hkv) { return Hkv >= 4 || Hkv <= 0 ? 1 : 4 / Hkv; }
-// The most of it that Hq query heads allow (Hkv >= Hq / 8): workspace queries
-// know Hq alone.
-int most_ranges(int Hq) { return kv_head_ranges((Hq + 7) / 8); }
+// Several ranges to a workgroup (1 or 2 kv heads) from as many tokens on as
+// give them work: 64 tokens of 512 to 8,192 keys at 4 / 1 heads 83 -> 49 us, at
+// 8 / 2 87 -> 77.5; 128 tokens over E4M3 at 4 / 1 heads 55 -> 44, at 8 / 2 66 ->
+// 60. Below, the longer search and the merge's extra records cost what the
+// bytes in flight gain: 48 tokens at 16 / 2 heads 45 -> 47 us, 35 short ones at
+// 4 / 1 24.8 -> 25.5, 1 token at 8 / 2 13.7 -> 14.5. Draft rows at 2 kv heads,
+// 4 records a piece, lose 4 % at every size.
+int ranges_per_wg(int T, int Hkv, bool f8, bool drafts) {
+    return T < (f8 && Hkv == 2 ? 128 : 64) || (drafts && Hkv == 2) ? 1 : kv_head_ranges(Hkv);
+}
+// Rows per segment and its records: vf_rows(G), which the 16 columns of one
+// MFMA hold; draft rows of a bf16 cache at G = 6 or 8 take two column blocks
+// for 4 rows to a page pass. 1: the decode kernels.
+int segment_rows(int G, bool f8, bool drafts) {
+    if (drafts) return !f8 && G >= 6 ? pkv::VF_ROWS : pkv::vf_rows(G);
+    return f8 || G == 4 ? 1 : pkv::vf_rows(G);
+}
 
 size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
@@ -89,8 +103,7 @@ struct DecodeLayout {
 };
 
 // Partial rows: (T + n_wg) indices x Hq heads x nr, 1 for the decode kernels
-// and the rows of a segment for the verify kernels (the workspace queries,
-// which do not know G, size for the most, VF_ROWS).
+// and the rows of a segment for the verify kernels.
 DecodeLayout decode_layout(int T, int Hq, int n_wg, int nr = 1) {
     DecodeLayout d;
     const size_t rows = (size_t)(T + n_wg) * Hq * nr;
@@ -477,18 +490,24 @@ int pkv_attn_decode_config(int wg_per_cu, int min_range) {
 
 int pkv_attn_decode_workspace(int T, int Hq, size_t* bytes) {
     if (T < 0 || Hq <= 0 || !bytes) return PKV_ERR_INVALID;
-    // Groups other than 4 query heads per kv head run the verify kernels'
-    // records, so the size covers both layouts.
-    const int n_wg = decode_n_wg() * F8_WG_PER_CU * most_ranges(Hq);
-    *bytes = std::max(decode_layout(T, Hq, n_wg).total, decode_layout(T, Hq, n_wg, pkv::VF_ROWS).total);
+    // One range per workgroup with the most records a piece, and what the
+    // several-range forms that T tokens of Hq heads can take need (more for 1
+    // kv head, up to 8 query heads, from 64 tokens on).
+    const int wgs = decode_n_wg();
+    size_t most = decode_layout(T, Hq, wgs * F8_WG_PER_CU, pkv::VF_ROWS).total;
+    for (int G = 1; G <= 8; G++) {
+        if (!supported_group(G) || Hq % G != 0) continue;
+        for (int f8 = 0; f8 < 2; f8++)
+            for (int drafts = 0; drafts < 2; drafts++) {
+                const int n_wg = wgs * (f8 ? F8_WG_PER_CU : 1) * ranges_per_wg(T, Hq / G, f8, drafts);
+                most = std::max(most, decode_layout(T, Hq, n_wg, segment_rows(G, f8, drafts)).total);
+            }
+    }
+    *bytes = most;
     return PKV_OK;
 }
 
-int pkv_attn_verify_workspace(int T, int Hq, size_t* bytes) {
-    if (T < 0 || Hq <= 0 || !bytes) return PKV_ERR_INVALID;
-    *bytes = decode_layout(T, Hq, decode_n_wg() * F8_WG_PER_CU * most_ranges(Hq), pkv::VF_ROWS).total;
-    return PKV_OK;
-}
+int pkv_attn_verify_workspace(int T, int Hq, size_t* bytes) { return pkv_attn_decode_workspace(T, Hq, bytes); }
 
 }  // extern "C"
 
@@ -548,22 +567,10 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
             return PKV_ERR_INVALID;
     }
     const int wgs = decode_n_wg() * (f8 ? F8_WG_PER_CU : 1);
-    // Several ranges to a workgroup (1 or 2 kv heads) from as many tokens on
-    // as give them work: 64 tokens of 512 to 8,192 keys at 4 / 1 heads 83 -> 49
-    // us, at 8 / 2 87 -> 77.5; 128 tokens over E4M3 at 4 / 1 heads 55 -> 44, at
-    // 8 / 2 66 -> 60. Below, the longer search and the merge's extra records
-    // cost what the bytes in flight gain: 48 tokens at 16 / 2 heads 45 -> 47
-    // us, 35 short ones at 4 / 1 24.8 -> 25.5, 1 token at 8 / 2 13.7 -> 14.5.
-    // Draft rows at 2 kv heads, 4 records a piece, lose 4 % at every size.
-    int rpb = T < (f8 && Hkv == 2 ? 128 : 64) || (drafts && Hkv == 2) ? 1 : kv_head_ranges(Hkv);
-    // Rows per segment and its records: vf_rows(G), which the 16 columns of one
-    // MFMA hold; draft rows at G = 6 or 8 take two column blocks for 4 rows to
-    // a page pass. (A workspace sized otherwise, as the no-allocation array,
-    // may not hold what is wanted.)
-    int nr = verify ? pkv::vf_rows(G) : 1;
-    if (drafts && !f8 && G >= 6 &&
-        workspace_bytes >= decode_layout(T, Hq, wgs * rpb, pkv::VF_ROWS).total)
-        nr = pkv::VF_ROWS;
+    // A workspace sized otherwise, as the no-allocation array, may not hold
+    // what is wanted: 2-row segments, one range per workgroup.
+    int rpb = ranges_per_wg(T, Hkv, f8, drafts), nr = segment_rows(G, f8, drafts);
+    if (workspace_bytes < decode_layout(T, Hq, wgs * rpb, nr).total && verify) nr = pkv::vf_rows(G);
     if (workspace_bytes < decode_layout(T, Hq, wgs * rpb, nr).total) rpb = 1;
     const int n_wg = wgs * rpb;
     const DecodeLayout lay = decode_layout(T, Hq, n_wg, nr);

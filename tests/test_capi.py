@@ -4,6 +4,8 @@ reaches a kernel."""
 import os
 import re
 
+import pytest
+
 import pkv
 
 HDR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include", "pkv.h")
@@ -73,6 +75,21 @@ def test_workspace_grows_with_tokens():
     a, b = pkv.attn_decode_workspace(1, 16), pkv.attn_decode_workspace(64, 16)
     assert b > a > 0
     assert (b - a) >= 63 * 16 * 256 * 4
+
+
+@pytest.mark.parametrize("T,Hq,ranges,rows", [
+    (8, 8, 512, 4), (63, 4, 512, 4), (64, 12, 512, 4), (300, 16, 512, 4), (200, 24, 512, 4), (0, 5, 512, 4),
+    (64, 8, 2048, 2), (64, 6, 2048, 2), (64, 4, 2048, 4), (128, 1, 2048, 4)])
+def test_workspace_holds_the_ranges_that_a_call_can_take(T, Hq, ranges, rows):
+    """256 CUs: two ranges per CU (an E4M3 cache) of 4 records each, and four
+    times the ranges only where one kv head (up to 8 query heads) and 64 tokens
+    can take them."""
+    up = lambda x: (x + 255) // 256 * 256
+    n = (T + ranges) * Hq * rows
+    if rows == 2:  # draft rows over a bf16 cache: half the ranges, twice the records
+        n = max(n, (T + ranges // 2) * Hq * 4)
+    want = up(4 * (T + 2)) + up(8 * n) + 1024 * n
+    assert pkv.attn_decode_workspace(T, Hq) == pkv.attn_verify_workspace(T, Hq) == want
 
 
 def test_reference_abi_code_object_exports_the_reference_kernel_names(tmp_path):
