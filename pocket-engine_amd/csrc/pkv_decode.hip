@@ -84,20 +84,21 @@ struct DecodeParams {
 constexpr int PAGE = 16;
 
 // Exclusive prefix sum over the block; returns the block total in `total`.
-__device__ __forceinline__ int block_scan(int v, int* sh, int& total) {
+template <class S>
+__device__ __forceinline__ S block_scan(S v, S* sh, S& total) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    int x = v;
+    S x = v;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
+        const S y = __shfl_up(x, o, 64);
         if (lane >= o) x += y;
     }
     if (lane == 63) sh[w] = x;
     __syncthreads();
-    int before = 0;
+    S before = 0;
     total = 0;
     for (int k = 0; k < nw; k++) {
-        const int s = sh[k];
+        const S s = sh[k];
         if (k < w) before += s;
         total += s;
     }
@@ -667,35 +668,44 @@ struct StepAppend {
     }
 };
 
+// What find_range scans: a token's keys.
+struct TokenKeys {
+    using Sum = int;
+    __device__ __forceinline__ int total(Sum W, int n_wg) { return W; }  // of the whole step, from its scan's sum
+    __device__ __forceinline__ int of(Sum v) const { return v; }
+    __device__ __forceinline__ int flag() const { return 0; }  // in offs[T + 1]
+};
+
 // The wave's key range [start, end) of the flattened key space (keys of token
-// t: lenf(t)), cut into at most p.n_wg equal ranges of R >= max(min_range,
-// ceil(W / n_wg)) keys, and the token t0 holding key `start` at offset off0.
-// The first workgroup also writes offs[t] (exclusive offsets), offs[T] = W
-// and offs[T + 1] = R (| rflag) for the merge. For T <= block size one scan serves
-// both; otherwise a first pass totals W and a second finds the offsets.
-// Called by the whole workgroup; returns false for a wave (or the whole
-// workgroup) whose range is empty. sh_t0: 2 ints per range of the workgroup.
-template <bool MULTI, class LenF>
-__device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWave<MULTI>& rw, LenF lenf, int* sh_scan,
-                                           int* sh_t0, int& start, int& end, int& t0, int& off0,
-                                           int rflag = 0) {
+// t: lenf(t), as `keys` reads it), cut into at most p.n_wg equal ranges of R >=
+// max(min_range, ceil(W / n_wg)) keys, and the token t0 holding key `start` at
+// offset off0. The first workgroup also writes offs[t] (exclusive offsets),
+// offs[T] = W and offs[T + 1] = R | keys.flag() for the merge. For T <= block
+// size one scan serves both; otherwise a first pass totals W and a second finds
+// the offsets. Called by the whole workgroup; returns false for a wave (or the
+// whole workgroup) whose range is empty. sh_t0: 2 ints per range of the
+// workgroup.
+template <bool MULTI, class LenF, class Keys>
+__device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWave<MULTI>& rw, LenF lenf, Keys& keys,
+                                           typename Keys::Sum* sh_scan, int* sh_t0, int& start, int& end, int& t0,
+                                           int& off0) {
+    using Sum = typename Keys::Sum;
     const int T = p.T, nthr = blockDim.x, tid = threadIdx.x, b = blockIdx.x;
     const bool writer = b == 0 && blockIdx.y == 0;
     const bool one = T <= nthr;
-    int W = 0, myL = 0, myoff = 0;
+    Sum sum = 0, mine = 0, before = 0;
     if (one) {
-        myL = tid < T ? lenf(tid) : 0;
-        myoff = block_scan(myL, sh_scan, W);
+        mine = tid < T ? lenf(tid) : 0;
+        before = block_scan(mine, sh_scan, sum);
     } else {
         for (int base = 0; base < T; base += nthr) {
             const int t = base + tid;
-            const int L = t < T ? lenf(t) : 0;
-            int tot;
-            block_scan(L, sh_scan, tot);
-            W += tot;
+            Sum tot;
+            block_scan(t < T ? lenf(t) : Sum(0), sh_scan, tot);
+            sum += tot;
         }
     }
-    W = __builtin_amdgcn_readfirstlane(W);  // block-uniform: keep it in scalar registers
+    const int W = __builtin_amdgcn_readfirstlane(keys.total(sum, p.n_wg));  // block-uniform: scalar registers
     int R = max(p.min_range, (W + p.n_wg - 1) / p.n_wg);
     if constexpr (MULTI) R = max(R, min(RANGE_KEYS, (W + p.nb - 1) / p.nb));
     // the workgroup's k-th range starts at key at(k) (W: past the last)
@@ -705,7 +715,7 @@ __device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWav
     end = range_end(start, R, W);
     if (writer && tid == 0) {
         p.offs[T] = W;
-        p.offs[T + 1] = R | rflag;
+        p.offs[T + 1] = R | keys.flag();
     }
     // token t at `off` with L keys: the workgroup's ranges that start in it
     auto mark = [&](int t, int off, int L) {
@@ -720,22 +730,22 @@ __device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWav
     };
     if (one) {
         if (tid < T) {
-            if (writer) p.offs[tid] = myoff;
-            mark(tid, myoff, myL);
+            if (writer) p.offs[tid] = keys.of(before);
+            mark(tid, keys.of(before), keys.of(mine));
         }
     } else {
         if (first >= W && b != 0) return false;
         int run = 0;
         for (int base = 0; base < T; base += nthr) {
             const int t = base + tid;
-            const int L = t < T ? lenf(t) : 0;
-            int tot;
-            const int off = run + block_scan(L, sh_scan, tot);
+            const Sum L = t < T ? lenf(t) : Sum(0);
+            Sum tot;
+            const int off = run + keys.of(block_scan(L, sh_scan, tot));
             if (t < T) {
                 if (writer) p.offs[t] = off;
-                mark(t, off, L);
+                mark(t, off, keys.of(L));
             }
-            run += tot;
+            run += keys.of(tot);
             if (b != 0 && run > last) break;  // uniform: every thread has the same run
         }
     }
@@ -771,6 +781,7 @@ __global__ void __launch_bounds__(256, 1)
     StepAppend<MULTI> app(rw);
     if constexpr (FUSED) app.begin(p, slot_map);
     int start, end, t0, off0;
+    TokenKeys keys;
     const bool any = find_range(
         p, rw,
         [&](int t) {
@@ -781,7 +792,7 @@ __global__ void __launch_bounds__(256, 1)
             }
             return L;
         },
-        sh_scan, sh_t0, start, end, t0, off0);
+        keys, sh_scan, sh_t0, start, end, t0, off0);
     if constexpr (FUSED) app.finish(p, slot_map);
     if (!any) return;
     const int wave = rw.wave, kvh = rw.kvh;

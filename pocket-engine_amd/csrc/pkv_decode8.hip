@@ -324,6 +324,7 @@ __global__ void __launch_bounds__(256, 2)
     const int b = rw.b;
     const bool tab = T <= nthr;
     int start, end, t0, off0;
+    TokenKeys keys;
     const bool any = find_range(
         p, rw,
         [&](int t) {
@@ -334,7 +335,7 @@ __global__ void __launch_bounds__(256, 2)
             }
             return L;
         },
-        sh_scan, sh_t0, start, end, t0, off0);
+        keys, sh_scan, sh_t0, start, end, t0, off0);
     if (!any) return;
     const int wave = rw.wave, kvh = rw.kvh;
     int t = t0, off = off0;

@@ -46,17 +46,16 @@ __host__ __device__ constexpr int vf_rows(int G) { return G <= 4 ? 4 : 2; }
 constexpr int VF_VSTR = HEAD_DIM + 16;    // u16 per staged V row (544 B: conflict-free transposed reads)
 constexpr int VF_LDS = PAGE * VF_VSTR;    // u16 per wave
 
-// Keys of the segment headed by token t (segments of NR rows, NR a power of
-// two); 0 when t does not head a segment (it is not at offset NR i of its
+// Keys of the segment headed by token t (segments of nr rows, nr a power of
+// two); 0 when t does not head a segment (it is not at offset nr i of its
 // sequence) or none of its rows attends.
-template <int NR>
-__device__ __forceinline__ int seg_len(int t, int T, const int* __restrict__ pos, const int* __restrict__ tok_seq,
+__device__ __forceinline__ int seg_len(int nr, int t, int T, const int* __restrict__ pos, const int* __restrict__ tok_seq,
                                        const int* __restrict__ cu, int skip, const int* __restrict__ outs, int spec,
                                        int& nrows) {
     const int s = tok_seq[t];
     nrows = 0;
-    if ((t - cu[s]) & (NR - 1)) return 0;
-    nrows = min(NR, min(cu[s + 1], T) - t);
+    if ((t - cu[s]) & (nr - 1)) return 0;
+    nrows = min(nr, min(cu[s + 1], T) - t);
     int L = 0;
     for (int r = 0; r < nrows; r++) L = max(L, decode_len(t + r, pos, tok_seq, cu, skip, outs, spec));
     return L;
@@ -96,9 +95,40 @@ struct SegTable {
 };
 
 // Two-block kernels: keys per range under which segments hold half the rows
-// (walk_segments), and the flag in offs[T + 1] that tells the merge.
+// (SegmentKeys), and the flag in offs[T + 1] that tells the merge.
 constexpr int SEG_HALF_KEYS = 96;
 constexpr int SEG_HALF_FLAG = 1 << 30;
+
+// What find_range scans for segments of NR rows: the keys of the segment that a
+// token heads.
+template <int NR, bool HALVES>
+struct SegmentKeys : TokenKeys {
+    static constexpr int rows = NR;
+    template <class F>
+    __device__ __forceinline__ Sum scan(F seg) const {
+        return seg(NR);
+    }
+};
+// HALVES (two column blocks): a short step, under SEG_HALF_KEYS keys a range,
+// takes NR / 2 rows to a segment: more and shorter segments, each of one block.
+// Both cuts go through the one scan, so that a step of any number of rows
+// decides without another: low word NR rows, high word NR / 2.
+template <int NR>
+struct SegmentKeys<NR, true> {
+    using Sum = unsigned long;
+    int rows = NR;
+    template <class F>
+    __device__ __forceinline__ Sum scan(F seg) const {
+        const Sum whole = (unsigned)seg(NR);
+        return whole | (Sum)(unsigned)seg(NR / 2) << 32;
+    }
+    __device__ __forceinline__ int total(Sum W, int n_wg) {
+        if (__builtin_amdgcn_readfirstlane((int)(unsigned)W) < SEG_HALF_KEYS * n_wg) rows = NR / 2;
+        return of(W);
+    }
+    __device__ __forceinline__ int of(Sum v) const { return (int)(unsigned)(rows < NR ? v >> 32 : v); }
+    __device__ __forceinline__ int flag() const { return rows < NR ? SEG_HALF_FLAG : 0; }
+};
 
 // One wave: segment headed by token t (rows t + r, r < NR, attending Lr[r]
 // keys; Lr = 0 for absent rows), kv head kvh with G query
@@ -358,41 +388,29 @@ struct VerifyEpi {
 // piece(t, nr, Lr, seq, row0, P0, j0, j1, direct): the segment headed by t (nr
 // rows, row r attending Lr[r] keys, of sequence seq whose first row is row0 at
 // position P0), keys [j0, j1) of the sequence, and whether they are all of the
-// segment's. before() runs between the search's loads and its end. HALVES (two
-// column blocks): a short step, under SEG_HALF_KEYS keys a range, takes NR / 2
-// rows to a segment: more and shorter segments, each of one block.
-template <int NR, bool HALVES, bool MULTI, class Before, class Piece>
-__device__ __forceinline__ void walk_segments(const DecodeParams& p, const RangeWave<MULTI>& rw, SegTable& tab,
-                                              int* sh_scan, int* sh_t0, const int* __restrict__ pos,
-                                              const int* __restrict__ tok_seq, const int* __restrict__ cu,
-                                              const int* __restrict__ outs, Before before, Piece piece) {
+// segment's. before() runs between the search's loads and its end.
+template <bool MULTI, class Keys, class Before, class Piece>
+__device__ __forceinline__ void walk_segments(const DecodeParams& p, const RangeWave<MULTI>& rw, Keys keys,
+                                              SegTable& tab, typename Keys::Sum* sh_scan, int* sh_t0,
+                                              const int* __restrict__ pos, const int* __restrict__ tok_seq,
+                                              const int* __restrict__ cu, const int* __restrict__ outs, Before before,
+                                              Piece piece) {
     const int T = p.T;
     const bool tabled = T <= SegTable::MAX;
     if (tabled) tab.fill(p, pos, tok_seq, cu, outs);
     int nr, start, end, t0, off0;
-    // rows per segment: NR, or NR / 2
-    int nrs = NR;
-    if constexpr (HALVES) {
-        if (tabled) {
-            int W;
-            for (int base = 0, run = W = 0; base < T; base += blockDim.x) {
-                const int t = base + threadIdx.x;
-                block_scan(t < T ? tab.seg_len(NR, t, nr) : 0, sh_scan, run);
-                W += run;
-            }
-            if (__builtin_amdgcn_readfirstlane(W) < SEG_HALF_KEYS * p.n_wg) nrs = NR / 2;
-        }
-    }
-    auto len_at = [&](int t) {
-        return tabled ? tab.seg_len(nrs, t, nr) : seg_len<NR>(t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr);
+    auto len_at = [&](int rows, int t) {
+        return tabled ? tab.seg_len(rows, t, nr)
+                      : seg_len(rows, t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr);
     };
-    const bool any = find_range(p, rw, len_at, sh_scan, sh_t0, start, end, t0, off0,
-                                nrs < NR ? SEG_HALF_FLAG : 0);
+    const bool any = find_range(
+        p, rw, [&](int t) { return keys.scan([&](int rows) { return len_at(rows, t); }); }, keys, sh_scan, sh_t0, start,
+        end, t0, off0);
     before();
     if (!any) return;
     int t = t0, off = off0;
     while (off < end && t < T) {
-        const int Ls = __builtin_amdgcn_readfirstlane(len_at(t));
+        const int Ls = __builtin_amdgcn_readfirstlane(len_at(keys.rows, t));
         nr = __builtin_amdgcn_readfirstlane(nr);
         if (Ls > 0) {
             int Lr[VF_ROWS], seq, row0, P0;
@@ -441,15 +459,16 @@ __global__ void __launch_bounds__(256, NR * G > 16 ? 1 : 2)
     verify_range_kernel(DecodeParams p, const int* __restrict__ pos, const int* __restrict__ tok_seq,
                         const int* __restrict__ block_table, const int* __restrict__ cu,
                         const int* __restrict__ outs, const int* __restrict__ slot_map) {
-    __shared__ int sh_scan[16];
+    using Keys = SegmentKeys<NR, (NR * G > 16)>;
+    __shared__ typename Keys::Sum sh_scan[4];
     __shared__ int sh_t0[8];
     __shared__ SegTable sh_tab;
     __shared__ __align__(16) uint16_t sh_v[4][VF_LDS];
     const RangeWave<MULTI> rw(p);
     StepAppend<MULTI> app(rw);
     if constexpr (FUSED) app.begin(p, slot_map);
-    walk_segments<NR, (NR * G > 16)>(
-        p, rw, sh_tab, sh_scan, sh_t0, pos, tok_seq, cu, outs,
+    walk_segments(
+        p, rw, Keys(), sh_tab, sh_scan, sh_t0, pos, tok_seq, cu, outs,
         [&]() {
             if constexpr (FUSED) app.finish(p, slot_map);
         },
@@ -480,8 +499,8 @@ __global__ void __launch_bounds__(256, 2)
     __shared__ SegTable sh_tab;
     __shared__ WaveLds8 sh_w8[4];
     const RangeWave<MULTI> rw(p);
-    walk_segments<NR, false>(
-        p, rw, sh_tab, sh_scan, sh_t0, pos, tok_seq, cu, outs, []() {},
+    walk_segments(
+        p, rw, SegmentKeys<NR, false>(), sh_tab, sh_scan, sh_t0, pos, tok_seq, cu, outs, []() {},
         [&](int t, int nr, const int(&Lr)[VF_ROWS], int seq, int row0, int P0, int j0, int j1, bool direct) {
             const VerifyEpi<G> vepi{p, t, rw.kvh, t + rw.b, direct};
             auto epi = [&](int c, int gq, const f32x4 (&acc)[16], float m, float l) {

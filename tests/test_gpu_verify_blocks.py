@@ -68,3 +68,26 @@ def test_small_workspace_and_skipped_prompts(dev, G, Hkv):
     assert (got[skipped] == 0x3333).all()
     ok, err = close(got[~skipped], want[~skipped])
     assert ok, f"max |diff| {err}"
+
+
+@pytest.mark.parametrize("G,Hkv,groups,halves", [
+    (6, 4, [(int(x), 4) for x in np.random.default_rng(8).integers(1, 90, 30)], True),      # within the table
+    (6, 2, [(int(x), 4) for x in np.random.default_rng(9).integers(1, 90, 80)], True),      # past it: 320 rows
+    (8, 1, [(300, 270), (40, 4), (9, 3), (70, 2)], True),                                   # a long draft run
+    (8, 4, [(int(x), 4) for x in np.random.default_rng(10).integers(400, 1000, 70)], False),  # past it, long
+    (6, 4, [(9000, 4), (7001, 3), (12000, 2), (8000, 5)], False)])
+def test_short_steps_take_half_segments_at_any_row_count(dev, G, Hkv, groups, halves):
+    """Under 96 keys a range, segments hold 2 rows, also where the step has more
+    rows than the segment table: the word behind the W of the workspace's
+    offsets tells the merge."""
+    print(f"case verify blocks halves={halves} G={G} Hkv={Hkv} ({len(groups)})", flush=True)
+    c = verify_case(groups, Hkv, 23, G=G)
+    T, Hq = c["T"], c["Hq"]
+    ws = torch.zeros(pkv.attn_verify_workspace(T, Hq), dtype=torch.uint8, device=dev)
+    out = torch.zeros(T, Hq, D, dtype=torch.int16, device=dev)
+    pkv.attn_verify(i16(c["q"], dev), i16(c["kc"], dev), i16(c["vc"], dev), i16(c["qkv"], dev), c["qstride"], Hq, Hkv,
+                    *[i32(c[k], dev) for k in ("pos", "tok_seq", "bt")], c["max_blocks"], BS, out, SCALE,
+                    i32(c["cu"], dev), 0, None, 1, T, c["pages"], ws)
+    ok, err = close(out.cpu().numpy().view(np.uint16), run_oracle(c))
+    assert ok, f"max |diff| {err}"
+    assert bool(ws.view(torch.int32)[T + 1].item() & 1 << 30) == halves
