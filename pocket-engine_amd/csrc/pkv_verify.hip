@@ -46,53 +46,29 @@ __host__ __device__ constexpr int vf_rows(int G) { return G <= 4 ? 4 : 2; }
 constexpr int VF_VSTR = HEAD_DIM + 16;    // u16 per staged V row (544 B: conflict-free transposed reads)
 constexpr int VF_LDS = PAGE * VF_VSTR;    // u16 per wave
 
-// Keys of the segment headed by token t (segments of nr rows, nr a power of
-// two); 0 when t does not head a segment (it is not at offset nr i of its
-// sequence) or none of its rows attends.
-__device__ __forceinline__ int seg_len(int nr, int t, int T, const int* __restrict__ pos, const int* __restrict__ tok_seq,
-                                       const int* __restrict__ cu, int skip, const int* __restrict__ outs, int spec,
-                                       int& nrows) {
+// Keys of the segment headed by token t (segments of nr <= VF_ROWS rows, a
+// power of two); 0 when t does not head a segment (it is not at offset nr i of
+// its sequence) or none of its rows attends. The rows are of one sequence, so
+// whether they attend is one answer, and their positions load beside tok_seq ->
+// cu, not row by row at the end of that chain: 8 sequences x 4 draft rows over
+// 400 keys, beside 300 prompt rows left out, at 16 / 2 heads 34.8 -> 23.9 us, at
+// 24 / 4 36.8 -> 29.3. (A table of the tokens in LDS, filled by the workgroup,
+// does not pay beside it: 100 x 4 rows over 300 keys at 12 / 2 heads 44.7 us
+// without, 45.9 with one.)
+__device__ __forceinline__ int seg_len(int nr, int t, int T, const int* __restrict__ pos,
+                                       const int* __restrict__ tok_seq, const int* __restrict__ cu, int skip,
+                                       const int* __restrict__ outs, int spec, int& nrows) {
     const int s = tok_seq[t];
-    nrows = 0;
-    if ((t - cu[s]) & (nr - 1)) return 0;
-    nrows = min(nr, min(cu[s + 1], T) - t);
+    int x[VF_ROWS];
+#pragma unroll
+    for (int r = 0; r < VF_ROWS; r++) x[r] = pos[min(t + r, T - 1)];
+    const int c0 = cu[s], c1 = cu[s + 1];
+    nrows = (t - c0) & (nr - 1) ? 0 : min(nr, min(c1, T) - t);
     int L = 0;
-    for (int r = 0; r < nrows; r++) L = max(L, decode_len(t + r, pos, tok_seq, cu, skip, outs, spec));
-    return L;
+#pragma unroll
+    for (int r = 0; r < VF_ROWS; r++) L = r < nrows ? max(L, x[r] + 1) : L;
+    return skip && c1 - c0 > 1 && !is_spec(outs, spec, s) ? 0 : L;
 }
-
-// What the verify kernels walk, in LDS for up to MAX tokens: per token its
-// attended keys, position, sequence, its row in the sequence and the rows left
-// from it on. Filled by the whole workgroup in two dependent round trips;
-// without it every segment met costs the chain tok_seq -> cu -> pos again (24
-// query heads, 1 sequence of 500 keys 14.9 -> 14.5 us, 200 of 40 to 2,500
-// 134.6 -> 133.5, 48 x 4 draft rows at 16 heads over 2,000 keys 26.0 -> 25.0).
-struct SegTable {
-    static constexpr int MAX = 256;
-    int len[MAX], pos[MAX], seq[MAX], rel[MAX], left[MAX];
-    __device__ __forceinline__ void fill(const DecodeParams& p, const int* __restrict__ pos_,
-                                         const int* __restrict__ tok_seq, const int* __restrict__ cu,
-                                         const int* __restrict__ outs) {
-        for (int t = threadIdx.x; t < p.T; t += blockDim.x) {
-            const int s = tok_seq[t], x = pos_[t];
-            const int c0 = cu[s], c1 = cu[s + 1];
-            const bool prompt = p.skip_prompts && c1 - c0 > 1 && !is_spec(outs, p.spec, s);
-            len[t] = prompt ? 0 : x + 1;
-            pos[t] = x;
-            seq[t] = s;
-            rel[t] = t - c0;
-            left[t] = min(c1, p.T) - t;
-        }
-        __syncthreads();
-    }
-    // Keys of the segment of nr rows headed by t, as seg_len.
-    __device__ __forceinline__ int seg_len(int nr, int t, int& nrows) const {
-        nrows = rel[t] & (nr - 1) ? 0 : min(nr, left[t]);
-        int L = 0;
-        for (int r = 0; r < nrows; r++) L = max(L, len[t + r]);
-        return L;
-    }
-};
 
 // Two-block kernels: keys per range under which segments hold half the rows
 // (SegmentKeys), and the flag in offs[T + 1] that tells the merge.
@@ -391,17 +367,13 @@ struct VerifyEpi {
 // segment's. before() runs between the search's loads and its end.
 template <bool MULTI, class Keys, class Before, class Piece>
 __device__ __forceinline__ void walk_segments(const DecodeParams& p, const RangeWave<MULTI>& rw, Keys keys,
-                                              SegTable& tab, typename Keys::Sum* sh_scan, int* sh_t0,
-                                              const int* __restrict__ pos, const int* __restrict__ tok_seq,
-                                              const int* __restrict__ cu, const int* __restrict__ outs, Before before,
-                                              Piece piece) {
+                                              typename Keys::Sum* sh_scan, int* sh_t0, const int* __restrict__ pos,
+                                              const int* __restrict__ tok_seq, const int* __restrict__ cu,
+                                              const int* __restrict__ outs, Before before, Piece piece) {
     const int T = p.T;
-    const bool tabled = T <= SegTable::MAX;
-    if (tabled) tab.fill(p, pos, tok_seq, cu, outs);
     int nr, start, end, t0, off0;
     auto len_at = [&](int rows, int t) {
-        return tabled ? tab.seg_len(rows, t, nr)
-                      : seg_len(rows, t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr);
+        return seg_len(rows, t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr);
     };
     const bool any = find_range(
         p, rw, [&](int t) { return keys.scan([&](int rows) { return len_at(rows, t); }); }, keys, sh_scan, sh_t0, start,
@@ -413,24 +385,13 @@ __device__ __forceinline__ void walk_segments(const DecodeParams& p, const Range
         const int Ls = __builtin_amdgcn_readfirstlane(len_at(keys.rows, t));
         nr = __builtin_amdgcn_readfirstlane(nr);
         if (Ls > 0) {
-            int Lr[VF_ROWS], seq, row0, P0;
-            if (tabled) {
+            int Lr[VF_ROWS];
 #pragma unroll
-                for (int r = 0; r < VF_ROWS; r++)
-                    Lr[r] = r < nr ? __builtin_amdgcn_readfirstlane(tab.len[t + r]) : 0;
-                seq = __builtin_amdgcn_readfirstlane(tab.seq[t]);
-                row0 = t - __builtin_amdgcn_readfirstlane(tab.rel[t]);
-                P0 = __builtin_amdgcn_readfirstlane(tab.pos[row0]);
-            } else {
-#pragma unroll
-                for (int r = 0; r < VF_ROWS; r++)
-                    Lr[r] = r < nr ? __builtin_amdgcn_readfirstlane(
-                                         decode_len(t + r, pos, tok_seq, cu, p.skip_prompts, outs, p.spec))
-                                   : 0;
-                seq = __builtin_amdgcn_readfirstlane(tok_seq[t]);
-                row0 = __builtin_amdgcn_readfirstlane(cu[seq]);
-                P0 = __builtin_amdgcn_readfirstlane(pos[row0]);
-            }
+            for (int r = 0; r < VF_ROWS; r++)
+                Lr[r] = r < nr ? __builtin_amdgcn_readfirstlane(pos[t + r]) + 1 : 0;  // (Ls > 0: the rows attend)
+            const int seq = __builtin_amdgcn_readfirstlane(tok_seq[t]);
+            const int row0 = __builtin_amdgcn_readfirstlane(cu[seq]);
+            const int P0 = __builtin_amdgcn_readfirstlane(pos[row0]);
             const int j0 = max(start, off) - off, j1 = min(end, off + Ls) - off;
             piece(t, nr, Lr, seq, row0, P0, j0, j1, j0 == 0 && j1 == Ls && !p.fo.mode);
             off += Ls;
@@ -462,13 +423,12 @@ __global__ void __launch_bounds__(256, NR * G > 16 ? 1 : 2)
     using Keys = SegmentKeys<NR, (NR * G > 16)>;
     __shared__ typename Keys::Sum sh_scan[4];
     __shared__ int sh_t0[8];
-    __shared__ SegTable sh_tab;
     __shared__ __align__(16) uint16_t sh_v[4][VF_LDS];
     const RangeWave<MULTI> rw(p);
     StepAppend<MULTI> app(rw);
     if constexpr (FUSED) app.begin(p, slot_map);
     walk_segments(
-        p, rw, Keys(), sh_tab, sh_scan, sh_t0, pos, tok_seq, cu, outs,
+        p, rw, Keys(), sh_scan, sh_t0, pos, tok_seq, cu, outs,
         [&]() {
             if constexpr (FUSED) app.finish(p, slot_map);
         },
@@ -496,11 +456,10 @@ __global__ void __launch_bounds__(256, 2)
     constexpr int NR = vf_rows(G);
     __shared__ int sh_scan[16];
     __shared__ int sh_t0[8];
-    __shared__ SegTable sh_tab;
     __shared__ WaveLds8 sh_w8[4];
     const RangeWave<MULTI> rw(p);
     walk_segments(
-        p, rw, SegmentKeys<NR, false>(), sh_tab, sh_scan, sh_t0, pos, tok_seq, cu, outs, []() {},
+        p, rw, SegmentKeys<NR, false>(), sh_scan, sh_t0, pos, tok_seq, cu, outs, []() {},
         [&](int t, int nr, const int(&Lr)[VF_ROWS], int seq, int row0, int P0, int j0, int j1, bool direct) {
             const VerifyEpi<G> vepi{p, t, rw.kvh, t + rw.b, direct};
             auto epi = [&](int c, int gq, const f32x4 (&acc)[16], float m, float l) {

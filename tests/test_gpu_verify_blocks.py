@@ -1,8 +1,8 @@
 """GPU parity of draft rows at 6 and 8 query heads per kv head, whose kernel
 takes 4 rows to a page pass in two column blocks (long steps), 2 rows to a
 pass (short steps), and one block for segments of up to 2 rows: row counts on
-every side of a segment, few and many keys per range, more rows than the
-segment table holds (256), prompt rows left out, and a workspace that holds
+every side of a segment, few and many keys per range, more rows than a
+workgroup has threads (256), prompt rows left out, and a workspace that holds
 only the 2-row records. Oracle at the bound of tests/_util.close."""
 import numpy as np
 import pytest
@@ -28,7 +28,7 @@ def default_config():
     (8, 2, [(33, 4), (129, 5), (64, 6), (1, 4)]),
     (6, 2, [(9000, 4), (7001, 3), (12000, 2), (8000, 5), (3, 4), (6500, 1)]),  # long: whole segments
     (8, 1, [(26000, 4), (15, 7), (3000, 2)]),
-    (6, 1, [(int(x), 4) for x in np.random.default_rng(3).integers(1, 900, 70)]),  # more rows than the table
+    (6, 1, [(int(x), 4) for x in np.random.default_rng(3).integers(1, 900, 70)]),  # more rows than threads
     (8, 4, [(int(x), 1 + i % 4) for i, x in enumerate(np.random.default_rng(4).integers(600, 1500, 30))])])
 def test_rows_match_oracle(dev, G, Hkv, groups):
     print(f"case verify blocks G={G} Hkv={Hkv} groups={groups[:6]} ({len(groups)})", flush=True)
@@ -71,14 +71,14 @@ def test_small_workspace_and_skipped_prompts(dev, G, Hkv):
 
 
 @pytest.mark.parametrize("G,Hkv,groups,halves", [
-    (6, 4, [(int(x), 4) for x in np.random.default_rng(8).integers(1, 90, 30)], True),      # within the table
-    (6, 2, [(int(x), 4) for x in np.random.default_rng(9).integers(1, 90, 80)], True),      # past it: 320 rows
+    (6, 4, [(int(x), 4) for x in np.random.default_rng(8).integers(1, 90, 30)], True),      # up to 256 rows
+    (6, 2, [(int(x), 4) for x in np.random.default_rng(9).integers(1, 90, 80)], True),      # 320 rows
     (8, 1, [(300, 270), (40, 4), (9, 3), (70, 2)], True),                                   # a long draft run
-    (8, 4, [(int(x), 4) for x in np.random.default_rng(10).integers(400, 1000, 70)], False),  # past it, long
+    (8, 4, [(int(x), 4) for x in np.random.default_rng(10).integers(400, 1000, 70)], False),  # 280 rows, long
     (6, 4, [(9000, 4), (7001, 3), (12000, 2), (8000, 5)], False)])
 def test_short_steps_take_half_segments_at_any_row_count(dev, G, Hkv, groups, halves):
     """Under 96 keys a range, segments hold 2 rows, also where the step has more
-    rows than the segment table: the word behind the W of the workspace's
+    rows than the workgroup threads: the word behind the W of the workspace's
     offsets tells the merge."""
     print(f"case verify blocks halves={halves} G={G} Hkv={Hkv} ({len(groups)})", flush=True)
     c = verify_case(groups, Hkv, 23, G=G)
