@@ -87,6 +87,14 @@ int kv_head_ranges(int Hkv) { return Hkv >= 4 || Hkv <= 0 ? 1 : 4 / Hkv; }
 int ranges_per_wg(int T, int Hkv, bool f8, bool drafts) {
     return T < (f8 && Hkv == 2 ? 128 : 64) || (drafts && Hkv == 2) ? 1 : kv_head_ranges(Hkv);
 }
+// T counts the rows of prompts that the call leaves out too. Over an E4M3 cache
+// at 2 kv heads, 1,024 ranges, a step where fewer than this many rows attend
+// takes one range per workgroup after all (0: never): 4 rows over 30,000 keys
+// beside a 512-row prompt at 8 / 2 heads 55.2 -> 47.8 us, 16 over 20,000 71.4 ->
+// 69.9. The others gain from the several ranges at few attending rows too: over
+// bf16 8 rows of 30,000 at 8 / 2 heads 101 us in one range, 96 in two, at 4 / 1
+// 99.8 and 61.5; over E4M3 16 of 20,000 at 4 / 1 61.8 and 54.1.
+int multi_rows(int Hkv, bool f8) { return f8 && Hkv == 2 ? 128 : 0; }
 // Rows per segment and its records: vf_rows(G), which the 16 columns of one
 // MFMA hold; draft rows of a bf16 cache at G = 6 or 8 take two column blocks
 // for 4 rows to a page pass. 1: the decode kernels.
@@ -598,6 +606,7 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
     p.part_acc = (float*)(ws + lay.acc);
     p.n_wg = n_wg;
     p.nb = wgs;
+    p.multi_rows = multi_rows(Hkv, f8);
     p.min_range = g_min_range;
     p.k_rows = app ? (const uint16_t*)app->k_rows : nullptr;
     p.v_rows = app ? (const uint16_t*)app->v_rows : nullptr;

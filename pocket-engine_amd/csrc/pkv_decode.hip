@@ -69,6 +69,7 @@ struct DecodeParams {
     float* part_acc;          // [(T + n_wg) * Hq][256]
     int n_wg, min_range;      // most key ranges, fewest keys of one
     int nb;                   // workgroups (RangeWave<true>)
+    int multi_rows;           // attending rows below which these take one range after all (skip_prompts)
     // fused step: the step's new rows (k_rows + t * row_stride, Hkv * 256 each)
     const uint16_t* k_rows;
     const uint16_t* v_rows;
@@ -677,14 +678,14 @@ struct TokenKeys {
 };
 
 // The wave's key range [start, end) of the flattened key space (keys of token
-// t: lenf(t), as `keys` reads it), cut into at most p.n_wg equal ranges of R >=
-// max(min_range, ceil(W / n_wg)) keys, and the token t0 holding key `start` at
-// offset off0. The first workgroup also writes offs[t] (exclusive offsets),
-// offs[T] = W and offs[T + 1] = R | keys.flag() for the merge. For T <= block
-// size one scan serves both; otherwise a first pass totals W and a second finds
-// the offsets. Called by the whole workgroup; returns false for a wave (or the
-// whole workgroup) whose range is empty. sh_t0: 2 ints per range of the
-// workgroup.
+// t: lenf(t, rows), as `keys` reads it, which adds t's attending rows to rows),
+// cut into at most p.n_wg equal ranges of R >= max(min_range, ceil(W / n_wg))
+// keys, and the token t0 holding key `start` at offset off0. The first workgroup
+// also writes offs[t] (exclusive offsets), offs[T] = W and offs[T + 1] = R |
+// keys.flag() for the merge. For T <= block size one scan serves both; otherwise
+// a first pass totals W and a second finds the offsets. Called by the whole
+// workgroup; returns false for a wave (or the whole workgroup) whose range is
+// empty. sh_t0: 2 ints per range of the workgroup.
 template <bool MULTI, class LenF, class Keys>
 __device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWave<MULTI>& rw, LenF lenf, Keys& keys,
                                            typename Keys::Sum* sh_scan, int* sh_t0, int& start, int& end, int& t0,
@@ -694,20 +695,31 @@ __device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWav
     const bool writer = b == 0 && blockIdx.y == 0;
     const bool one = T <= nthr;
     Sum sum = 0, mine = 0, before = 0;
+    int attending = 0;  // rows that attend, of those that this thread meets
     if (one) {
-        mine = tid < T ? lenf(tid) : 0;
+        mine = tid < T ? lenf(tid, attending) : 0;
         before = block_scan(mine, sh_scan, sum);
     } else {
         for (int base = 0; base < T; base += nthr) {
             const int t = base + tid;
             Sum tot;
-            block_scan(t < T ? lenf(t) : Sum(0), sh_scan, tot);
+            block_scan(t < T ? lenf(t, attending) : Sum(0), sh_scan, tot);
             sum += tot;
         }
     }
     const int W = __builtin_amdgcn_readfirstlane(keys.total(sum, p.n_wg));  // block-uniform: scalar registers
     int R = max(p.min_range, (W + p.n_wg - 1) / p.n_wg);
-    if constexpr (MULTI) R = max(R, min(RANGE_KEYS, (W + p.nb - 1) / p.nb));
+    if constexpr (MULTI) {
+        // (T counts the rows of prompts left out too)
+        const int per_wg = (W + p.nb - 1) / p.nb;
+        int least = min(RANGE_KEYS, per_wg);
+        if (p.multi_rows > 0 && p.skip_prompts && per_wg > RANGE_KEYS) {
+            Sum rows;
+            block_scan((Sum)attending, sh_scan, rows);
+            if ((int)rows < p.multi_rows) least = per_wg;
+        }
+        R = max(R, least);
+    }
     // the workgroup's k-th range starts at key at(k) (W: past the last)
     auto at = [&](int k) { return __builtin_amdgcn_readfirstlane(range_start(b + k * p.nb, R, W)); };
     const int first = at(0), last = MULTI ? at(rw.rpb - 1) : first;
@@ -738,7 +750,7 @@ __device__ __forceinline__ bool find_range(const DecodeParams& p, const RangeWav
         int run = 0;
         for (int base = 0; base < T; base += nthr) {
             const int t = base + tid;
-            const Sum L = t < T ? lenf(t) : Sum(0);
+            const Sum L = t < T ? lenf(t, attending) : Sum(0);
             Sum tot;
             const int off = run + keys.of(block_scan(L, sh_scan, tot));
             if (t < T) {
@@ -784,12 +796,13 @@ __global__ void __launch_bounds__(256, 1)
     TokenKeys keys;
     const bool any = find_range(
         p, rw,
-        [&](int t) {
+        [&](int t, int& rows) {
             const int L = decode_len(t, pos, tok_seq, cu, p.skip_prompts, outs, p.spec);
             if (tab) {
                 sh_pos[t] = pos[t];
                 sh_seq[t] = tok_seq[t];
             }
+            rows += L > 0;
             return L;
         },
         keys, sh_scan, sh_t0, start, end, t0, off0);

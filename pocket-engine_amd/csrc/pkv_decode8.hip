@@ -327,12 +327,13 @@ __global__ void __launch_bounds__(256, 2)
     TokenKeys keys;
     const bool any = find_range(
         p, rw,
-        [&](int t) {
+        [&](int t, int& rows) {
             const int L = decode_len(t, pos, tok_seq, cu, p.skip_prompts, outs, p.spec);
             if (tab) {
                 sh_pos[t] = pos[t];
                 sh_seq[t] = tok_seq[t];
             }
+            rows += L > 0;
             return L;
         },
         keys, sh_scan, sh_t0, start, end, t0, off0);

@@ -376,8 +376,14 @@ __device__ __forceinline__ void walk_segments(const DecodeParams& p, const Range
         return seg_len(rows, t, T, pos, tok_seq, cu, p.skip_prompts, outs, p.spec, nr);
     };
     const bool any = find_range(
-        p, rw, [&](int t) { return keys.scan([&](int rows) { return len_at(rows, t); }); }, keys, sh_scan, sh_t0, start,
-        end, t0, off0);
+        p, rw,
+        [&](int t, int& rows) {
+            int L;  // of the last cut, which holds every row once
+            const auto sum = keys.scan([&](int per_seg) { return L = len_at(per_seg, t); });
+            rows += L > 0 ? nr : 0;
+            return sum;
+        },
+        keys, sh_scan, sh_t0, start, end, t0, off0);
     before();
     if (!any) return;
     int t = t0, off = off0;

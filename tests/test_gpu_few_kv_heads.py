@@ -5,6 +5,7 @@ ranges shorter and longer than the least kept, sequences of one key, rows of
 prompts left out, against the oracle at the bound of tests/_util.close."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 import pkv
@@ -95,3 +96,39 @@ def test_noalloc_step(dev, G, Hkv, T):
     assert np.array_equal(kc, wkc) and np.array_equal(vc, wvc), "appended rows differ"
     ok, err = close(got, want)
     assert ok, f"max |diff| {err}"
+
+
+@pytest.mark.parametrize("G,Hkv,f8,prompt,rows,multi", [
+    (4, 2, True, 200, 100, False), (8, 2, True, 300, 127, False), (4, 2, True, 30, 128, True), (4, 1, True, 33, 70, True),
+    (4, 2, False, 200, 40, True), (8, 1, False, 90, 40, True)])
+def test_rows_that_attend_choose_the_ranges(dev, G, Hkv, f8, prompt, rows, multi):
+    """Over E4M3 at 2 kv heads a prompt left out by skip_prompts doesn't count
+    as rows that give a workgroup's several ranges work: the keys per range (the
+    word behind the offsets' last, W) are those of one range per workgroup."""
+    print(f"case few kv heads mixed G={G} Hkv={Hkv} f8={f8} prompt={prompt} rows={rows}", flush=True)
+    lens = [int(x) for x in np.random.default_rng(rows).integers(1000, 3000, rows)]
+    c = verify_case([(40, prompt)] + [(L, 1) for L in lens], Hkv, rows, G=G)
+    T, Hq = c["T"], c["Hq"]
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    bf = lambda k: t(c[k].view(np.int16))
+    meta = [t(c[k]) for k in ("pos", "tok_seq", "bt")]
+    out = torch.full((T, Hq, 256), 0x3333, dtype=torch.int16, device=dev)
+    ws = torch.zeros(pkv.attn_decode_workspace(T, Hq), dtype=torch.uint8, device=dev)
+    tail = [c["max_blocks"], BS, out, SCALE, t(c["cu"]), 1, None, 1, T, c["pages"], ws]
+    args = (c["qkv"], c["qstride"], Hq, Hkv, c["pos"], c["tok_seq"], c["bt"], c["max_blocks"], BS, SCALE)
+    if f8:
+        k8, v8, ks, vs = e4m3_of(c, np.random.default_rng(rows), 0.02)
+        pkv.attn_decode_e4m3(bf("q"), t(k8), t(v8), t(ks), t(vs), bf("qkv"), c["qstride"], Hq, Hkv, *meta, *tail)
+        want = oracle.attn_decode8(c["q"], k8, v8, ks, vs, *args, cu=c["cu"])
+    else:
+        pkv.attn_decode(bf("q"), bf("kc"), bf("vc"), bf("qkv"), c["qstride"], Hq, Hkv, *meta, *tail)
+        want = run_oracle_v(c)
+    got = out.cpu().numpy().view(np.uint16)
+    assert (got[:prompt] == 0x3333).all()
+    ok, err = close(got[prompt:], want[prompt:])
+    assert ok, f"max |diff| {err}"
+    W, R = ws.view(torch.int32)[T:T + 2].tolist()
+    assert W == sum(lens) + rows
+    nb = torch.cuda.get_device_properties(0).multi_processor_count * (2 if f8 else 1)
+    per_wg = -(-W // nb)
+    assert R == (max(32, -(-W // (nb * 4 // Hkv)), min(128, per_wg)) if multi else max(32, per_wg))
