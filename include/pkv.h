@@ -100,8 +100,8 @@ int pkv_mtp_next(const int32_t* rows, const int32_t* pos, const int32_t* rope, i
  * G = Hq / Hkv in {1, 2, 4, 6, 8})
  * ------------------------------------------------------------------------- */
 
-/* Workspace bytes pkv_attn_decode needs for T tokens and Hq query heads on
- * the current device. */
+/* Workspace bytes that pkv_attn_decode, pkv_attn_verify and their E4M3 forms
+ * take for up to T tokens and Hq query heads on the current device. */
 int pkv_attn_decode_workspace(int T, int Hq, size_t* bytes);
 
 /* Paged decode attention with the reference's semantics and arguments
@@ -176,11 +176,14 @@ int pkv_attn_decode_step(const void* k_rows, const void* v_rows, int64_t row_str
  * forbid hipMalloc). It has no counterpart in the reference. The workspace is a
  * file-scope device array of PKV_NOALLOC_SCRATCH_BYTES per GPU; the call
  * allocates nothing (no hipMalloc / hipFree, no allocating library routine).
- * Same arguments and results as pkv_attn_decode_step otherwise. Returns
- * PKV_ERR_UNSUPPORTED when the step's workspace exceeds the array:
+ * Same arguments as pkv_attn_decode_step otherwise, and the same results bit
+ * for bit where both cut the keys into the same ranges; with 1 or 2 kv heads
+ * and 64 tokens or more a workspace of the queried size holds 4 / Hkv times as
+ * many ranges, which the array does not at some shapes (the sums then differ in
+ * their last bits). Returns PKV_ERR_UNSUPPORTED when the step's workspace with
+ * the fewest ranges exceeds the array:
  * 256-aligned (T + 2) int32 offsets, then (T + R) * Hq * n partial rows of
- * 2 + 256 f32 (R = key ranges = CUs x pkv_attn_decode_config's wg_per_cu;
- * n = 1 for G = 4, else the verify kernel's rows per segment: 4 for G <= 4,
+ * 2 + 256 f32 (R = CUs x pkv_attn_decode_config's wg_per_cu; n = 1 for G = 4, else the verify kernel's rows per segment: 4 for G <= 4,
  * 2 for G = 6 or 8); on a 256-CU device T <= 759 at Hq = 16 (G = 4) and
  * T <= 82 at Hq = 24 (G = 6). Every call on one GPU shares that GPU's array, so calls that
  * overlap on one GPU (different streams, or host threads) race; calls in

@@ -254,7 +254,8 @@ int pkv_attn_prep(const void* qkv, int qstride, int Hq, int Hkv, const float* q_
     }
     // Units (pairs of heads) per wave: 4 once that still leaves 8,192 waves
     // (the cos / sin of a token are evaluated fewer times: 8,192 rows at
-    // 16 / 4 heads 50.9 -> 44.9 us, 2,048 at 24 / 4 19.6 -> 17.0), else 1,
+    // 16 / 4 heads 50.9 us with 1, 44.9 with 4 in that run, 2,048 at 24 / 4
+    // 19.6 and 17.0), else 1,
     // which fills the chip sooner and has one pass to wait for (64 rows 3.0
     // against 4.4 us, 512 rows 5.5 against 6.4).
     const pkv::PrepPairs pairs(Hq, Hkv);
@@ -663,7 +664,7 @@ int attn_decode_phases(int phases, const AppendArgs* app, const float* kscale, c
         // Waves per (token, head) block: 16 when there are fewer blocks than
         // CUs (a head's records, up to one per range, load in one round), as
         // 4 blocks of 64 dims while those still fit the CUs (the whole step of
-        // 1 sequence of 4,096 keys 15.1 -> 13.7 us, of 60,000 over E4M3 45.7 ->
+        // 1 sequence of 4,096 keys 14.9 -> 13.3 us, of 60,000 over E4M3 45.7 ->
         // 40.1, 4 sequences 24.9 -> 24.2; with 128 such blocks 0.5 us slower,
         // with 192 or more 3 to 10 %); one
         // when a token has at most 12 records on average ((T + n_wg) / T: one

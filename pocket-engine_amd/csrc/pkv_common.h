@@ -71,8 +71,10 @@ __device__ __forceinline__ float gated_div(float x, float y) {
     const float c = __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
     return __builtin_isinf(y) ? 0.f * x : c;
 }
-// Two finite floats to packed bf16 with the hardware's round-to-nearest-even
-// conversion (one v_cvt_pk_bf16_f32); for values that are never NaN.
+// Two floats to packed bf16 with the hardware's round-to-nearest-even conversion
+// (one v_cvt_pk_bf16_f32). Denormals and infinities convert as in f2b_bits; a
+// NaN stays a NaN, of the hardware's payload (tests/test_gpu_gate_edges.py,
+// tests/test_gpu_prep.py hold them).
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack2_hw(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){lo, hi}, bf16x2));

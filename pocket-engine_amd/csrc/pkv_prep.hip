@@ -23,7 +23,7 @@
 // (DPP, one permlane swap), a rotary pair's partner (d + 32) sits 4 lanes
 // away inside the same 16-lane row and moves as packed bf16.
 // What bounds it: for prompts HBM (8,192 rows at 16 / 4 heads, 201 MB:
-// 44.6 us, 4.5 TB/s, where a 2 GiB device copy reaches 4.9; 141.9 us with a
+// 43.9 us, 4.6 TB/s, where a 2 GiB device copy reaches 4.9; 142.3 us with a
 // wave per head, 4 dims per lane and 8 cos / sin evaluations per lane and
 // wave, which was bound by VALU issue); for decode steps the launch and one
 // dependent round trip (64 rows 5.0 -> 3.0 us).
